@@ -28,11 +28,10 @@ def reference_logits(model, ids):
     """fp32 forward over one full sequence with the engine's weights; returns
     logits [T, vocab].  The restatement (oracle.qwen3_ref) is pinned to
     transformers' Qwen3 in tests/test_oracle_pins.py."""
-    key = id(model)
-    if key not in _REFS:
+    if _REFS.get("model") is not model:  # the object itself: a freed model's id is reused
         _REFS.clear()
-        _REFS[key] = Qwen3Ref.from_model(model)
-    return _REFS[key].logits(ids)
+        _REFS.update(model=model, ref=Qwen3Ref.from_model(model))
+    return _REFS["ref"].logits(ids)
 
 
 def _prompts(n, seed):
