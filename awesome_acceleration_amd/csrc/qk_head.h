@@ -17,8 +17,10 @@ template <Dt DT> struct Cvt;
 template <> struct Cvt<Dt::BF16> {
   __device__ static inline float lo(u32 w) { return bf16lo(w); }
   __device__ static inline float hi(u32 w) { return bf16hi(w); }
-  __device__ static inline u32 pack(float a, float b) { return pack_bf16x2(a, b); }
-  __device__ static inline float round(float x) { return __uint_as_float(f32_to_bf16_bits(x) << 16); }
+  // v_cvt_pk_bf16_f32 (round to nearest even): the same bits as
+  // f32_to_bf16_bits for every number, a fifth of its instructions
+  __device__ static inline u32 pack(float a, float b) { return Elem<Dt::BF16>::pack2_hw(a, b); }
+  __device__ static inline float round(float x) { return bf16lo(pack(x, x)); }
 };
 template <> struct Cvt<Dt::FP16> {
   __device__ static inline float lo(u32 w) { return f16lo(w); }
