@@ -27,13 +27,6 @@ constexpr int64_t kQkTokenKernelMin = 4096;
 
 namespace fz {
 
-__device__ __forceinline__ float wave_sum(float x) {
-  x = row16_sum(x);
-  x += __shfl_xor(x, 16);
-  x += __shfl_xor(x, 32);
-  return x;
-}
-
 // ---------------------------------------------------------------- RMSNorm
 // One wavefront per row; lane owns 8 consecutive elements per 512-element
 // chunk.  With a residual: h = x + residual (rounded), residual_out = h.

@@ -34,6 +34,7 @@
 // land on one XCD (workgroups are dealt round-robin over the 8 XCDs), so a
 // W tile is fetched from HBM once per XCD and re-read from that XCD's L2.
 
+#include "gemm_small.h"
 #include "qk_head.h"
 
 namespace aac {
@@ -371,6 +372,22 @@ extern "C" int aac_gemm_nt(const void* x, int64_t x_row_stride, const void* w, i
   if (((uintptr_t)x | (uintptr_t)w) % 16 || (uintptr_t)y % 8 || x_row_stride % 8 ||
       w_row_stride % 8 || y_row_stride % 4)
     return AAC_ERR_MISALIGNED;
+  if (config == 0 && gs::small_takes(m, n, k)) {
+    gs::Args s{};
+    s.x = (const u16*)x;
+    s.w = (const u16*)w;
+    s.y = (u16*)y;
+    s.x_stride = x_row_stride;
+    s.w_stride = w_row_stride;
+    s.y_stride = y_row_stride;
+    s.m = m;
+    s.k = k;
+    s.silu_off = silu_intermediate;
+    const int rc = gs::launch_small(s, n, silu, dtype == AAC_DTYPE_FP16, (hipStream_t)stream);
+    if (rc != AAC_OK) return rc;
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? AAC_OK : (int)e;
+  }
   const int cfg = config ? config : gm::pick_config(m, n, k);
   if (cfg == 0) return AAC_ERR_UNSUPPORTED;
   const int tc = 32 * gm::kCfg[cfg][1];

@@ -45,6 +45,13 @@ __device__ __forceinline__ u32x4 pack8(const float* f) {
   return w;
 }
 
+__device__ __forceinline__ float wave_sum(float x) {
+  x = row16_sum(x);
+  x += __shfl_xor(x, 16);
+  x += __shfl_xor(x, 32);
+  return x;
+}
+
 // ------------------------------------------------- q/k RMSNorm + RoPE + store
 struct QkArgs {
   const u16* qkv;

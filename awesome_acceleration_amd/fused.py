@@ -10,7 +10,7 @@ import torch
 from . import _lib
 
 __all__ = ["rmsnorm", "qk_norm_rope_store", "qkv_norm_rope_store", "silu_mul", "linear",
-           "linear_supported", "rmsnorm_supported", "argmax"]
+           "linear_supported", "rmsnorm_supported", "rmsnorm_linear", "argmax"]
 
 
 def _stream(t: torch.Tensor) -> int:
@@ -159,6 +159,41 @@ def linear(x: torch.Tensor, weight: torch.Tensor, silu: bool = False,
                                 _code(x), _stream(x))
     _lib.check(rc, "aac_gemm_nt")
     return y
+
+
+def _norm_args(x, weight, w, residual):
+    """(m, k, residual_out) of a norm-fused projection's arguments, checked."""
+    _req(x.is_cuda and x.dim() == 2 and x.stride(1) == 1, "x must be a [rows, hidden] GPU tensor")
+    m, k = x.shape
+    _req(weight.shape == (k,) and weight.dtype == x.dtype and weight.is_contiguous(), "norm weight")
+    _req(w.dim() == 2 and w.stride(1) == 1 and w.dtype == x.dtype and w.shape[1] == k,
+         "projection weight must be [n, hidden] with contiguous rows, same dtype as x")
+    if residual is None:
+        return m, k, None
+    _req(residual.shape == x.shape and residual.is_contiguous() and residual.dtype == x.dtype,
+         "residual shape")
+    return m, k, torch.empty_like(residual)
+
+
+def _ptr(t: Optional[torch.Tensor]):
+    return t.data_ptr() if t is not None else None
+
+
+def rmsnorm_linear(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, weight: torch.Tensor,
+                   residual: Optional[torch.Tensor] = None, silu: bool = False):
+    """``linear(rmsnorm(x, norm_weight, eps, residual), weight, silu)`` in one
+    launch for a decode step of few rows (hidden 512 or 1024).  Returns
+    ``(y, x + residual)``; the second is ``None`` without a residual."""
+    m, k, res_out = _norm_args(x, norm_weight, weight, residual)
+    n = weight.shape[0] // 2 if silu else weight.shape[0]
+    _req(not silu or weight.shape[0] == 2 * n, "gate/up weight must have an even row count")
+    y = torch.empty((m, n), dtype=x.dtype, device=x.device)
+    rc = _lib.lib().aac_rmsnorm_gemm_nt(
+        x.data_ptr(), x.stride(0), _ptr(residual), _ptr(res_out), norm_weight.data_ptr(), float(eps),
+        weight.data_ptr(), weight.stride(0), y.data_ptr(), y.stride(0), m, n, k, n if silu else 0,
+        _code(x), _stream(x))
+    _lib.check(rc, "aac_rmsnorm_gemm_nt")
+    return y, res_out
 
 
 def linear_supported(m: int, n: int, k: int) -> bool:

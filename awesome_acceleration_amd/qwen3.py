@@ -39,6 +39,9 @@ from . import paged
 __all__ = ["Qwen3Config", "Qwen3ForCausalLM", "PagedKVCache", "StepMeta"]
 
 
+NORM_GEMM_ROWS = 16
+
+
 @dataclass
 class Qwen3Config:
     """Same fields and defaults as the reference's Qwen3Config (model/model.py:13-37)."""
@@ -175,6 +178,9 @@ class Qwen3ForCausalLM:
         if self.d != 128 or H % 128 or not all(fz.linear_supported(1, n, k) for n, k in (
                 (self.q_size + 2 * self.kv_size, H), (H, self.q_size), (I, H), (H, I))):
             self.small_gemm_rows = 0  # a shape the decode-batch GEMM has no tiling for
+        # up to this many sequences the residual add and RMSNorm before a
+        # projection run in the projection's own launch
+        self.norm_gemm_rows = NORM_GEMM_ROWS if self.small_gemm_rows and H in (512, 1024) else 0
         self.rope = Rope(self.d, cfg.max_position_embeddings, cfg.rope_theta, self.device, dtype)
 
     @torch.no_grad()
@@ -263,6 +269,7 @@ class Qwen3ForCausalLM:
         pos = meta.positions if meta.positions.dtype == torch.int32 else meta.positions.int()
         small = not prefill and T <= self.small_gemm_rows
         lin = fz.linear if small else F.linear
+        merged = small and T <= self.norm_gemm_rows
         for li, L in enumerate(self.layers):
             if delta is None:
                 x = fz.rmsnorm(res, L["ln1"], eps)
@@ -294,6 +301,10 @@ class Qwen3ForCausalLM:
                                         meta.context_lens, softmax_scale=self.scale,
                                         max_context_len=meta.max_context_len)
             o = lin(attn.reshape(T, -1), L["o"])
+            if merged:
+                act, res = fz.rmsnorm_linear(o, L["ln2"], eps, L["gate_up"], residual=res, silu=True)
+                delta = fz.linear(act, L["down"])
+                continue
             x, res = fz.rmsnorm(o, L["ln2"], eps, residual=res)
             if small:
                 delta = fz.linear(fz.linear(x, L["gate_up"], silu=True), L["down"])

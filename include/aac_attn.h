@@ -343,6 +343,18 @@ int aac_qkv_norm_rope_store(const void* x, int64_t x_row_stride, const void* w_q
                             void* stream);
 
 /*
+ * aac_gemm_nt with the residual add and RMSNorm of aac_rmsnorm in its
+ * prologue, for a decode step of few rows: h = x, or h = dtype(x + residual)
+ * with residual_out = h when residual is given (both contiguous [m, k]; not
+ * the same buffer), y = norm(h) w^T (with silu_intermediate: SiLU * up).  k is
+ * 512 or 1024 and n a multiple of 32, else AAC_ERR_UNSUPPORTED.
+ */
+int aac_rmsnorm_gemm_nt(const void* x, int64_t x_row_stride, const void* residual,
+                        void* residual_out, const void* norm_weight, float eps, const void* w,
+                        int64_t w_row_stride, void* y, int64_t y_row_stride, int32_t m, int32_t n,
+                        int32_t k, int32_t silu_intermediate, int32_t dtype, void* stream);
+
+/*
  * Greedy sampling: out[r] = the index of the largest element of row r of x
  * [n_rows, n_cols] (row stride row_stride elements; BF16, FP16 or FP32), the
  * first one among equal maxima, a NaN counting as the largest -- the result

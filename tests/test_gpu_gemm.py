@@ -120,3 +120,35 @@ def test_rejects_bad_arguments(gpu):
         fz.linear(x, torch.zeros((64, 1000), device=gpu, dtype=torch.bfloat16))
     with pytest.raises(RuntimeError):
         fz.linear(x.float(), w.float())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m", [1, 8, 9, 16, 17, 32, 33, 64, 65])
+@pytest.mark.parametrize("n,k", [(1024, 512), (2048, 1024), (32, 3584), (2016, 3072)])
+def test_few_rows_match_fp32_reference(gpu, m, n, k, dtype):
+    """The small-batch kernel at the edges of its row tiles and column widths,
+    at depths of one unit per wave to more than fit LDS, with strided rows."""
+    x, w = _inputs(gpu, m, n, k, dtype, seed=m + n + k, x_pad=8, w_pad=16)
+    y = fz.linear(x, w)
+    torch.cuda.synchronize()
+    _check_linear(y, x, w, f"{m}x{n}x{k} {dtype}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m", [1, 8, 13, 16, 40])
+@pytest.mark.parametrize("n,k,silu", [(96, 512, False), (4096, 1024, False), (3072, 1024, True)])
+def test_norm_in_the_projection_equals_norm_then_projection(gpu, m, n, k, silu, dtype):
+    """aac_rmsnorm_gemm_nt normalises in the RMSNorm kernel's order and sums in
+    the small-batch projection's, so the two launches give the same bits."""
+    x, w = _inputs(gpu, m, 2 * n if silu else n, k, dtype, seed=m + n, x_pad=8)
+    g = torch.Generator(device=gpu).manual_seed(m)
+    res = torch.randn((m, k), generator=g, device=gpu).to(dtype)
+    nw = (1 + 0.3 * torch.randn(k, generator=g, device=gpu)).to(dtype)
+    for r in (None, res):
+        y, h = fz.rmsnorm_linear(x, nw, 1e-6, w, residual=r, silu=silu)
+        ref = fz.rmsnorm(x, nw, 1e-6, residual=r)
+        xn, href = (ref, None) if r is None else ref
+        want = torch.cat([fz.linear(xn[i:i + 32], w, silu=silu) for i in range(0, m, 32)])
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
+        assert h is None if r is None else torch.equal(h, href)
