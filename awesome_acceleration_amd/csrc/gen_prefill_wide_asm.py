@@ -35,7 +35,7 @@ together.
 
 Register map (fixed, clobbered):
   v152-v167 S0, v168-v183 S1     scores of column 0 / 1 (32 keys x 32 queries)
-  v184-v191 P0, v192-v199 P1     bf16 probabilities, two 16-key steps each
+  v184-v191 P0, v192-v199 P1     16-bit probabilities, two 16-key steps each
   v200-v203 L0, v204-v207 L1     row sums (16x16x32 selector MFMA layout)
   v208-v215 KA                   K read addresses (one per 16-dim step), tile t+1
   v216-v219 VA, v220-v223 VB     V read addresses (one per 32-dim block), tiles t, t+1
@@ -148,8 +148,12 @@ def VF_half(vset, f, h):
 LAYOUT = "early2"
 PARTIAL = True
 
-MFMA = "v_mfma_f32_32x32x16_bf16"
-SELM = "v_mfma_f32_16x16x32_bf16"
+# The template is a macro of the element type, "bf16" or "f16": both have the
+# same MFMA shapes, cycles and operand layouts and a round-to-nearest-even pack.
+TY = "{TY}"
+MFMA = f"v_mfma_f32_32x32x16_{TY}"
+SELM = f"v_mfma_f32_16x16x32_{TY}"
+CVT = f"v_cvt_pk_{TY}_f32"
 
 
 class Emitter:
@@ -245,7 +249,7 @@ def softmax_ops(x):
     steps = [[] for _ in range(18)]
     fma = lambda i: f"v_fma_f32 {S_e(x, i)}, {S_e(x, i)}, %[cs], {v(NB[x])}"
     ex = lambda i: f"v_exp_f32 {S_e(x, i)}, {S_e(x, i)}"
-    cvt = lambda w: f"v_cvt_pk_bf16_f32 {P_e(x, w)}, {S_e(x, 2 * w)}, {S_e(x, 2 * w + 1)}"
+    cvt = lambda w: f"{CVT} {P_e(x, w)}, {S_e(x, 2 * w)}, {S_e(x, 2 * w + 1)}"
     if LAYOUT == "base":
         for i in range(16):
             steps[i].append(fma(i))
@@ -741,7 +745,7 @@ def generate() -> str:
         for t in range(8):
             e(q_load(c, t))
     e("Lqdone_%=:")
-    # (4) O / l rounded to bf16, through this wave's LDS staging rows (beside
+    # (4) O / l rounded to 16 bits, through this wave's LDS staging rows (beside
     # the ring: 32 rows x 128 bytes at a 136-byte pitch, one half of a column
     # at a time) to whole 128-byte row segments in global memory.  Lane l
     # holds query l % 32, dims 32 db + 8 i + 4 (l / 32) + 0..3 of register
@@ -783,8 +787,8 @@ def generate() -> str:
                     e(f"v_mul_f32 {v(KA + i)}, {v(KA + i)}, {inv}")
                 pb = P[db % 2]
                 for r in range(4):
-                    e(f"v_cvt_pk_bf16_f32 {v(pb + 2 * r)}, {v(KA + 4 * r)}, {v(KA + 4 * r + 1)}")
-                    e(f"v_cvt_pk_bf16_f32 {v(pb + 2 * r + 1)}, {v(KA + 4 * r + 2)}, {v(KA + 4 * r + 3)}")
+                    e(f"{CVT} {v(pb + 2 * r)}, {v(KA + 4 * r)}, {v(KA + 4 * r + 1)}")
+                    e(f"{CVT} {v(pb + 2 * r + 1)}, {v(KA + 4 * r + 2)}, {v(KA + 4 * r + 3)}")
                 for r in range(4):
                     e(f"ds_write_b64 %[stw], {vr(pb + 2 * r, 2)} offset:{64 * (db % 2) + 16 * r}")
             # rows 8 i + l / 8, bytes 16 (l % 8) of the half
@@ -846,11 +850,12 @@ HEADER = """// Generated by gen_prefill_wide_asm.py -- do not edit by hand.
 
 def render() -> str:
     body = generate()
-    lit = "\n".join('  "' + ln.replace('"', '\\"') + '\\n"' for ln in body.split("\n"))
+    lit = "\n".join('  "' + ln.replace('"', '\\"').replace(TY, '" TY "') + '\\n"'
+                    for ln in body.split("\n"))
     n = sum(1 for ln in body.split("\n") if ln and not ln.endswith(":"))
     clob = ", ".join([f'"v{i}"' for i in VGPR_CLOBBER] + [f'"a{i}"' for i in AGPR_CLOBBER] +
                      [f'"s{i}"' for i in SGPR_CLOBBER] + ['"vcc"', '"m0"', '"scc"', '"memory"'])
-    return (HEADER + f"// {n} instructions.\n#define AAC_PW_ITEM_ASM \\\n" + " \\\n".join(lit.split("\n")) +
+    return (HEADER + f"// {n} instructions.\n#define AAC_PW_ITEM_ASM(TY) \\\n" + " \\\n".join(lit.split("\n")) +
             "\n\n#define AAC_PW_CLOBBERS " + clob + "\n")
 
 

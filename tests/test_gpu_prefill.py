@@ -397,3 +397,28 @@ def test_split_prefills_on_two_streams_keep_their_own_workspaces(gpu):
         assert torch.equal(o2, alone[1]), f"stream 2, round {rnd}"
     keys = {k for k in fai._pf_ws if k[0] == gpu.index or gpu.index is None}
     assert {s1.cuda_stream, s2.cuda_stream} <= {k[1] for k in keys}
+
+
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (32, 8), (32, 4)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_prefill_tile_edges_plain_and_stored(gpu, hq, hkv, dtype):
+    # enough segments that the persistent kernel takes the call; lengths on
+    # both sides of its 32-, 64- and 128-row edges; with the store the output
+    # is the same bit for bit and the caches hold the rows
+    print(f"case: tile edges {hq}/{hkv} {dtype}", flush=True)
+    lens = [1, 31, 32, 33, 63, 64, 65, 127, 128, 129, 200, 257] * 8
+    q, k, v, cq, _ = _ragged(lens, lens, hq, hkv, dtype, gpu, 31)
+    out = fai.flash_attn_varlen_func(q, k, v, cq, cq, 257, 257, causal=True)
+    n = sum(lens)
+    kc = torch.zeros((-(-n // 64) + 1, 64, hkv, 128), dtype=dtype, device=gpu)
+    vc = torch.zeros_like(kc)
+    slots = torch.randperm(kc.shape[0] * 64, device=gpu)[:n].to(torch.int64)
+    out2 = fai.varlen_prefill_with_kvcache(q, k, v, cq, 257, kc, vc, slots, causal=True)
+    torch.cuda.synchronize()
+    assert torch.equal(out, out2)
+    assert torch.equal(kc.view(-1, hkv, 128)[slots], k) and torch.equal(vc.view(-1, hkv, 128)[slots], v)
+    m = sum(lens[:12])
+    cu = cq.cpu().numpy()[:13]
+    ref = oracle.varlen_attention(f64(q[:m]), f64(k[:m]), f64(v[:m]), cu, scale=128 ** -0.5)
+    absv = oracle.varlen_attention(f64(q[:m]), f64(k[:m]), np.abs(f64(v[:m])), cu, scale=128 ** -0.5)
+    check_attention(out[:m], ref, what="tile edges", absv=absv)
