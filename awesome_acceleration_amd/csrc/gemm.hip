@@ -255,7 +255,7 @@ __global__ __launch_bounds__(64 * MW * NW * KS) void gemm_kernel(Args a) {
       const int p = fz::clamp_pos(q, q.positions[t]);
       fz::unpack8<DT>(*reinterpret_cast<const u32x4*>((hh < q.hq ? q.qw : q.kw) + li * 8), wf);
       fz::unpack8<DT>(*reinterpret_cast<const u32x4*>(q.cos + (int64_t)p * kHeadDimFused + li * 8), cf);
-      fz::unpack8<DT>(*reinterpret_cast<const u32x4*>(q.sin + (int64_t)p * kHeadDimFused + li * 8), sf);
+      fz::signed_sin<DT>(q.sin + (int64_t)p * kHeadDimFused + li * 8, li, sf);
     }
     fz::norm_rope_head<DT>(q, t, hh, li, xr, crow, wf, cf, sf);
     return;

@@ -45,6 +45,26 @@ __device__ __forceinline__ u32x4 pack8(const float* f) {
   return w;
 }
 
+// Both values rounded to the activation type: one convert and two unpacks.
+template <Dt DT>
+__device__ __forceinline__ void round2(float& a, float& b) {
+  const u32 w = Cvt<DT>::pack(a, b);
+  a = Cvt<DT>::lo(w);
+  b = Cvt<DT>::hi(w);
+}
+
+// 16 bytes to memory; NT: non-temporal, past the caches.
+template <bool NT> __device__ __forceinline__ void put16(u16* p, const u32x4& w) {
+  if constexpr (NT) __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(p));
+  else *reinterpret_cast<u32x4*>(p) = w;
+}
+
+// 16 bytes read once; NT: non-temporal.
+template <bool NT> __device__ __forceinline__ u32x4 get16(const u16* p) {
+  if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+  else return *reinterpret_cast<const u32x4*>(p);
+}
+
 __device__ __forceinline__ float wave_sum(float x) {
   x = row16_sum(x);
   x += __shfl_xor(x, 16);
@@ -102,7 +122,9 @@ __device__ __forceinline__ int64_t cache_row(const QkArgs& a, int64_t t) {
 // (model/model.py:90-99); rotate_half pairs dim d with d +- 64, i.e. lane li
 // with lane li ^ 8 (DPP row_ror:8).  The caller keeps the row's 16 lanes
 // together on every branch.
-template <Dt DT>
+// sf holds sin with the sign of rotate_half folded in: negative in the lanes
+// of the first half (li < 8), see signed_sin.
+template <Dt DT, bool NT = false>
 __device__ __forceinline__ void norm_rope_head(const QkArgs& a, int64_t t, int hh, int li,
                                                const u32x4& xr, int64_t crow, const float* wf,
                                                const float* cf, const float* sf) {
@@ -112,8 +134,7 @@ __device__ __forceinline__ void norm_rope_head(const QkArgs& a, int64_t t, int h
 #pragma clang fp contract(off)
   if (hh >= a.hq + a.hkv) {  // value head
     if (crow >= 0)
-      *reinterpret_cast<u32x4*>(a.v_cache + (crow * a.hkv + (hh - a.hq - a.hkv)) * kHeadDimFused +
-                                li * 8) = xr;
+      put16<NT>(a.v_cache + (crow * a.hkv + (hh - a.hq - a.hkv)) * kHeadDimFused + li * 8, xr);
     return;
   }
   float x[8];
@@ -124,25 +145,44 @@ __device__ __forceinline__ void norm_rope_head(const QkArgs& a, int64_t t, int h
   ss = row16_sum(ss);
   const float rs = __frsqrt_rn(ss / (float)kHeadDimFused + a.eps);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) x[i] = Cvt<DT>::round(wf[i] * Cvt<DT>::round(x[i] * rs));
-  float o[8];
+  for (int i = 0; i < 8; ++i) x[i] *= rs;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float partner = __int_as_float(
-        __builtin_amdgcn_update_dpp(0, __float_as_int(x[i]), 0x128, 0xF, 0xF, false));
-    const float rot = li < 8 ? -partner : partner;
-    o[i] = Cvt<DT>::round(Cvt<DT>::round(x[i] * cf[i]) + Cvt<DT>::round(rot * sf[i]));
+  for (int i = 0; i < 8; i += 2) round2<DT>(x[i], x[i + 1]);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) x[i] *= wf[i];
+#pragma unroll
+  for (int i = 0; i < 8; i += 2) round2<DT>(x[i], x[i + 1]);
+  u32x4 packed;
+#pragma unroll
+  for (int i = 0; i < 8; i += 2) {
+    float c[2], r[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const float partner = __int_as_float(
+          __builtin_amdgcn_update_dpp(0, __float_as_int(x[i + e]), 0x128, 0xF, 0xF, false));
+      c[e] = x[i + e] * cf[i + e];
+      r[e] = partner * sf[i + e];
+    }
+    round2<DT>(c[0], c[1]);
+    round2<DT>(r[0], r[1]);
+    packed[i / 2] = Cvt<DT>::pack(c[0] + r[0], c[1] + r[1]);
   }
-  const u32x4 packed = pack8<DT>(o);
   if (hh < a.hq) {
-    *reinterpret_cast<u32x4*>(a.q_out + (t * a.hq + hh) * kHeadDimFused + li * 8) = packed;
+    put16<NT>(a.q_out + (t * a.hq + hh) * kHeadDimFused + li * 8, packed);
   } else {
     const int kh = hh - a.hq;
-    if (a.k_out != nullptr)
-      *reinterpret_cast<u32x4*>(a.k_out + (t * a.hkv + kh) * kHeadDimFused + li * 8) = packed;
-    if (crow >= 0)
-      *reinterpret_cast<u32x4*>(a.k_cache + (crow * a.hkv + kh) * kHeadDimFused + li * 8) = packed;
+    if (a.k_out != nullptr) put16<NT>(a.k_out + (t * a.hkv + kh) * kHeadDimFused + li * 8, packed);
+    if (crow >= 0) put16<NT>(a.k_cache + (crow * a.hkv + kh) * kHeadDimFused + li * 8, packed);
   }
+}
+
+// sin of the lane's dims, negated in the first half: rounding is symmetric,
+// so (-partner) * sin and partner * (-sin) are the same bits.
+template <Dt DT>
+__device__ __forceinline__ void signed_sin(const u16* sin8, int li, float* sf) {
+  unpack8<DT>(*reinterpret_cast<const u32x4*>(sin8), sf);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) sf[i] = li < 8 ? -sf[i] : sf[i];
 }
 
 __device__ __forceinline__ int clamp_pos(const QkArgs& a, int p) {
