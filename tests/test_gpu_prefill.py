@@ -422,3 +422,48 @@ def test_prefill_tile_edges_plain_and_stored(gpu, hq, hkv, dtype):
     ref = oracle.varlen_attention(f64(q[:m]), f64(k[:m]), f64(v[:m]), cu, scale=128 ** -0.5)
     absv = oracle.varlen_attention(f64(q[:m]), f64(k[:m]), np.abs(f64(v[:m])), cu, scale=128 ** -0.5)
     check_attention(out[:m], ref, what="tile edges", absv=absv)
+
+
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (16, 4), (16, 2)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("causal", [True, False])
+def test_prefill_few_queries(gpu, hq, hkv, dtype, causal):
+    # few items: the keys split over a workgroup's waves.  Query counts around
+    # the 32-row blocks, key counts around the 32-key sub-tiles and the 128-key
+    # iterations, more and fewer keys than queries, empty segments, strided rows
+    print(f"case: few queries {hq}/{hkv} {dtype} causal={causal}", flush=True)
+    lq = [1, 31, 33, 64, 0, 5, 40, 32]
+    lk = [1, 31, 33, 129, 7, 600, 11, 0]
+    q, k, v, cq, ck = _ragged(lq, lk, hq, hkv, dtype, gpu, 41)
+    wide = torch.randn((sum(lk), 2 * hkv + 1, 128), device=gpu).to(dtype)
+    wide[:, 1:hkv + 1], wide[:, hkv + 1:] = k, v
+    k, v = wide[:, 1:hkv + 1], wide[:, hkv + 1:]
+    out = fai.flash_attn_varlen_func(q, k, v, cq, ck, max(lq), max(lk), causal=causal)
+    torch.cuda.synchronize()
+    cu_q, cu_k = cq.cpu().numpy(), ck.cpu().numpy()
+    ref = oracle.varlen_attention(f64(q), f64(k), f64(v), cu_q, cu_seqlens_k=cu_k,
+                                  scale=128 ** -0.5, causal=causal)
+    absv = oracle.varlen_attention(f64(q), f64(k), np.abs(f64(v)), cu_q, cu_seqlens_k=cu_k,
+                                   scale=128 ** -0.5, causal=causal)
+    check_attention(out, ref, what="few queries", absv=absv)
+    if not causal:
+        return
+    # with the store: same output, every token stored, a padding slot and a
+    # max_seqlen below the longest segment (its first rows have no item)
+    lens = [70, 3, 33]
+    q, k, v, cq, _ = _ragged(lens, lens, hq, hkv, dtype, gpu, 43)
+    n = sum(lens)
+    slots = torch.randperm(256, device=gpu)[:n].to(torch.int64)
+    slots[2] = -1
+    for most in (70, 40):
+        kc = torch.zeros((4, 64, hkv, 128), dtype=dtype, device=gpu)
+        vc = torch.zeros_like(kc)
+        plain = fai.flash_attn_varlen_func(q, k, v, cq, cq, most, most, causal=True)
+        stored = fai.varlen_prefill_with_kvcache(q, k, v, cq, most, kc, vc, slots, causal=True)
+        torch.cuda.synchronize()
+        keep = slots >= 0
+        ek, ev = torch.zeros_like(kc).view(-1, hkv, 128), torch.zeros_like(vc).view(-1, hkv, 128)
+        ek[slots[keep]], ev[slots[keep]] = k[keep], v[keep]
+        assert torch.equal(kc.view(-1, hkv, 128), ek) and torch.equal(vc.view(-1, hkv, 128), ev)
+        if most == 70:
+            assert torch.equal(plain, stored)
