@@ -38,6 +38,13 @@
 //   type and P.V is v_dot2 over V words paired across two tokens (v_perm);
 //   fp32: unpacked fp32 FMAs with q pre-scaled.  The 16 row states of a workgroup are
 //   merged at the end (cross-row shuffles inside a wave, LDS across waves).
+//
+// The new token (aac_decode_append_paged, aac_decode_qkv_paged): appended by
+// the attention launch itself, see NEW at the kernel.  Against a store launch
+// before it: 24 slot-layout sequences of 100-2063 tokens 29.5 -> 26.5 us a call, a
+// 28-layer step of 4 sequences 935 -> 881 (with the q/k norm + RoPE folded in
+// too); 256 x 1-2k the same (240.8 and 240.9).
+//
 //   A sequence whose context spans one partition writes the final output
 //   directly; longer contexts write a normalised partial output and its
 //   log-sum-exp to the workspace, and a second kernel combines the
@@ -51,7 +58,8 @@
 #include <climits>
 #include <mutex>
 
-#include "aac_common.h"
+#include "qk_head.h"
+
 
 namespace aac {
 
@@ -87,7 +95,24 @@ struct DecodeArgs {
   int32_t bs_mshift;
   int32_t lpt;       // 1: blockIdx.z is a rank in descending context order
   int32_t lpt_max;   // context bound the length classes are scaled to
+  // The new token's rows of sequence b (NEW): [n_seqs, hkv, 128] with these
+  // sequence strides (elements); lens[b] is its position.  The caches are
+  // written here.
+  const void* k_new;
+  const void* v_new;
+  int64_t k_new_stride, v_new_stride;
+  // NEW == kQkv: q and k_new are the projection's raw rows; norm weights, RoPE
+  // tables [max_pos, 128] and positions as in qk_head.h
+  const u16 *qw, *kw, *cos, *sin;
+  const int32_t* positions;
+  int32_t max_pos;
+  float eps;
 };
+
+// What the launch does with the step's new token: nothing (its rows are in the
+// caches already), append its K/V rows, or also make q and k from the QKV
+// projection's rows (q/k RMSNorm + RoPE).
+enum { kNone = 0, kAppend = 1, kQkv = 2 };
 
 // Raw storage for the 8 elements one lane owns in one token row.
 template <Dt DT> struct Raw8 {
@@ -101,6 +126,10 @@ template <Dt DT> struct Raw8 {
   __device__ inline void zero() {
 #pragma unroll
     for (int i = 0; i < kWords; ++i) w[i] = u32x4{0, 0, 0, 0};
+  }
+  __device__ inline void store(char* p) const {
+#pragma unroll
+    for (int i = 0; i < kWords; ++i) *reinterpret_cast<u32x4*>(p + 16 * i) = w[i];
   }
   __device__ inline void unpack(float* f) const {
     if constexpr (DT == Dt::FP32) {
@@ -204,7 +233,11 @@ __device__ __forceinline__ void store_out2(void* out, int64_t idx, float x0, flo
   }
 }
 
-template <Dt DT, int G, int U, bool POW2>
+// NEW: the workgroup that holds the new token (the last one of the context)
+// starts its online softmax from it, straight from the given rows, and writes
+// them to the caches: the loop is that of kNone, and there is no launch before
+// this one.
+template <Dt DT, int G, int U, bool POW2, int NEW>
 // Occupancy: with G <= 2 the kernel fits 128 VGPRs, i.e. four workgroups per
 // CU (16 wavefronts); larger groups hold more accumulators.
 __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(DecodeArgs a) {
@@ -226,6 +259,7 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
                      : (int)blockIdx.z;  // wave-uniform (SGPR) either way
   const int ctx = context_len(a, b);
   const int np = parts_of(a, ctx);
+  constexpr int R = 16;  // token rows of the workgroup (one per DPP row)
 
   if (part >= np) {
     if (part == 0) {  // empty context: zeros (FA2 convention)
@@ -238,11 +272,30 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
     return;
   }
   const int t0 = part * a.part_tokens;
-  const int t1 = (part == np - 1) ? ctx : t0 + a.part_tokens;
+  int t1 = (part == np - 1) ? ctx : t0 + a.part_tokens;
 
   const int lane = tid & 63, wave = tid >> 6;
   const int li = lane & 15, grp = lane >> 4;
-  const int rslot = wave * 4 + grp;  // 0..15
+  const int rslot = wave * 4 + grp;  // 0 .. R - 1
+
+  // NEW == kQkv: norm + rotation of one head row.  `dim` is opaque, so that the
+  // new key's use of the norm and RoPE rows at the end of the loop reads them
+  // again instead of holding them in registers through it.
+  auto new_head = [&](const u32x4& raw, const u16* w) {
+    u32x4 o = raw;
+    if constexpr (NEW == kQkv) {
+      int dim = li * 8;
+      asm volatile("" : "+v"(dim));
+      const int pos = a.positions[b];
+      const int64_t p = (int64_t)(pos < 0 ? 0 : (pos >= a.max_pos ? a.max_pos - 1 : pos)) * kHeadDim + dim;
+      float wf[8], cf[8], sf[8];
+      fz::unpack8<DT>(*reinterpret_cast<const u32x4*>(w + dim), wf);
+      fz::unpack8<DT>(*reinterpret_cast<const u32x4*>(a.cos + p), cf);
+      fz::signed_sin<DT>(a.sin + p, li, sf);
+      o = fz::norm_rope_row<DT>(raw, a.eps, wf, cf, sf);
+    }
+    return o;
+  };
 
   // q for the G heads of this KV head.  fp32: unpacked and pre-scaled into
   // the log2 domain.  bf16/fp16 (PK): kept packed and exact for v_dot2; the
@@ -257,6 +310,9 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
     for (int g = 0; g < G; ++g) {
       Raw8<DT> r;
       r.load(qb + (int64_t)g * kHeadDim * ES);
+      if constexpr (NEW == kQkv) {
+        r.w[0] = new_head(r.w[0], a.qw);
+      }
       if constexpr (PK) {
 #pragma unroll
         for (int w = 0; w < 4; ++w) qp[g][w] = r.w[0][w];
@@ -294,16 +350,61 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
   // with in-order load counters, also wait for every K/V load issued before
   // it and leave one token per wave in flight.
   int blk[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) blk[u] = bt[block_index(token(t0 + rslot + 16 * u))];
 
-  for (int tb = t0 + rslot; tb < t1; tb += 16 * U) {
+  // NEW: the last partition's first row starts from the new token, whose K and V
+  // it also writes to the caches; the loop ends before it.  Not appended past
+  // the table or to a block outside the cache (the loop then reads what the
+  // caches hold, as for kNone).
+  if constexpr (NEW != kNone) {
+    const int pos = a.lens[b];
+    if (part == np - 1 && pos == ctx - 1) {
+      const int bi = block_index(pos), bk = bt[bi];
+      if ((uint32_t)bk < nb32) {
+        t1 = pos;
+        if (wave == 0) {
+          Raw8<DT> kx, vx;
+          kx.load(reinterpret_cast<const char*>(a.k_new) + ((int64_t)b * a.k_new_stride + (int64_t)h * kHeadDim + li * 8) * ES);
+          vx.load(reinterpret_cast<const char*>(a.v_new) + ((int64_t)b * a.v_new_stride + (int64_t)h * kHeadDim + li * 8) * ES);
+          if constexpr (NEW == kQkv) kx.w[0] = new_head(kx.w[0], a.kw);
+          float vf[8], kf[PK ? 1 : 8];
+          vx.unpack(vf);
+          if constexpr (!PK) kx.unpack(kf);
+          const bool first = lane < kRowLanes;
+#pragma unroll
+          for (int g = 0; g < G; ++g) {
+            float d = 0.f;
+            if constexpr (PK) {
+#pragma unroll
+              for (int w = 0; w < 4; ++w) d = Elem<DT>::dot2(kx.w[0][w], qp[g][w], d);
+            } else {
+#pragma unroll
+              for (int i = 0; i < 8; ++i) d = fmaf(qf[g][i], kf[i], d);
+            }
+            d = row16_sum(d);
+            m[g] = first ? (PK ? d * a.scale_log2 : d) : m[g];
+            l[g] = first ? 1.f : 0.f;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) acc[g][i] = first ? vf[i] : 0.f;
+          }
+          if (first) {
+            const int64_t off = ((int64_t)bk * a.block_size + (pos - bi * a.block_size)) * tok_bytes;
+            kx.store(const_cast<char*>(kbase) + off);
+            vx.store(const_cast<char*>(vbase) + off);
+          }
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) blk[u] = bt[block_index(token(t0 + rslot + R * u))];
+
+  for (int tb = t0 + rslot; tb < t1; tb += R * U) {
     Raw8<DT> kr[U], vr[U];
     bool valid[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      valid[u] = tb + 16 * u < t1;
-      const int t = token(tb + 16 * u);
+      valid[u] = tb + R * u < t1;
+      const int t = token(tb + R * u);
       const int bi = block_index(t);
       const int off = POW2 ? t & (a.block_size - 1) : t - bi * a.block_size;
       const uint32_t bk = (uint32_t)blk[u] < nb32 ? (uint32_t)blk[u] : 0u;  // bad entries read block 0
@@ -312,7 +413,7 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
       vr[u].load(vbase + row * tok_bytes);
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u) blk[u] = bt[block_index(token(tb + 16 * U + 16 * u))];
+    for (int u = 0; u < U; ++u) blk[u] = bt[block_index(token(tb + R * U + R * u))];
     // Every load above is issued before any arithmetic below (the scheduler
     // would otherwise pull each token's math up behind its load and wait).
     __builtin_amdgcn_sched_barrier(0);
@@ -472,22 +573,51 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
 
 // Combine the partitions of every (sequence, query head) whose context was
 // split: out = sum_p 2^(lse_p - LSE) o_p with LSE = log2 sum_p 2^lse_p.
+// Four wavefronts per (sequence, query head): each finds the largest lse (one
+// load per 64 partitions), then wave w sums partitions w, w + 4, ... with four
+// in flight, and the four sums meet in LDS.  The chain of loads is what it
+// costs: one wave walking the partitions one by one took 5.2 us at 11 partitions
+// of 24 sequences.
 template <Dt DT>
-__global__ __launch_bounds__(64) void decode_reduce_kernel(DecodeArgs a) {
+__global__ __launch_bounds__(256) void decode_reduce_kernel(DecodeArgs a) {
   const int hq = blockIdx.x, b = blockIdx.y;
   const int np = parts_of(a, context_len(a, b));
   if (np <= 1) return;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t slot0 = ((int64_t)b * a.hq + hq) * a.n_parts;
   float mx = -INFINITY;
-  for (int p = 0; p < np; ++p) mx = fmaxf(mx, a.ws_lse[slot0 + p]);
+  for (int p = lane; p < np; p += 64) mx = fmaxf(mx, a.ws_lse[slot0 + p]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
   float W = 0.f, o0 = 0.f, o1 = 0.f;
-  for (int p = 0; p < np; ++p) {
-    const float w = fast_exp2(a.ws_lse[slot0 + p] - mx);
-    const float2 o = *reinterpret_cast<const float2*>(a.ws_o + (slot0 + p) * kHeadDim + 2 * lane);
-    W += w;
-    o0 = fmaf(w, o.x, o0);
-    o1 = fmaf(w, o.y, o1);
+  for (int p = wave; p < np; p += 16) {
+    float lse[4];
+    float2 o[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t slot = slot0 + min(p + 4 * u, np - 1);
+      lse[u] = a.ws_lse[slot];
+      o[u] = *reinterpret_cast<const float2*>(a.ws_o + slot * kHeadDim + 2 * lane);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float w = p + 4 * u < np ? fast_exp2(lse[u] - mx) : 0.f;
+      W += w;
+      o0 = fmaf(w, o[u].x, o0);
+      o1 = fmaf(w, o[u].y, o1);
+    }
+  }
+  __shared__ float sw[4];
+  __shared__ float2 so[4][64];
+  so[wave][lane] = make_float2(o0, o1);
+  if (lane == 0) sw[wave] = W;
+  __syncthreads();
+  if (wave) return;
+#pragma unroll
+  for (int w = 1; w < 4; ++w) {
+    W += sw[w];
+    o0 += so[w][lane].x;
+    o1 += so[w][lane].y;
   }
   const float inv = 1.f / W;
   store_out2<DT>(a.out, (int64_t)b * a.out_seq_stride + (int64_t)hq * kHeadDim + 2 * lane, o0 * inv,
@@ -502,25 +632,37 @@ struct DecodePlan {
 };
 
 static DecodePlan plan_decode(int32_t n_seqs, int32_t hq, int32_t hkv, int32_t block_size,
-                              int32_t max_blocks, int32_t max_context_len, int32_t part_tokens) {
+                              int32_t max_blocks, int32_t max_context_len, int32_t part_tokens,
+                              int32_t elem_bytes) {
+  // tokens of one iteration of a workgroup: 16 rows x 8 in flight (fp32: 4)
+  const int iter_tokens = elem_bytes == 4 ? 64 : 128;
   DecodePlan p;
   int64_t cap = (int64_t)max_blocks * block_size;
   if (max_context_len > 0 && max_context_len < cap) cap = max_context_len;
   if (cap < 1) cap = 1;
   int64_t part = part_tokens;
   if (part <= 0) {
-    // Measured on MI355X (bf16, block 256): with >= 1024 (sequence, KV head)
-    // items and contexts up to 4096 tokens one workgroup per item streams at
-    // the HBM ceiling and needs no reduction; otherwise 3072-token partitions
-    // (64 x 16k-32k GQA-4 over four context draws: 75.4% of HBM peak against
-    // 73.8% for 2048, 75.1% for 2560, 74.3% for 3584 and 72.5% for 4096),
-    // halved until there are >= 2048 workgroups for 256 CUs.
+    // Measured on MI355X (block 256, graph replay, us).  From 512 (sequence, KV
+    // head) items and contexts up to 4096 tokens one workgroup per item needs no
+    // reduction and is the fastest (64 x 1-2k at 8 KV heads 66.7 against 68.3-73
+    // in partitions of 128-1024; 64 x 10-200 10.8 against 13.9-16.3), and up to
+    // two iterations of tokens for any number (1 x 93: 4.9 against 6.2).  Else the
+    // smallest partition, from one iteration up, that keeps the tables' capacity
+    // within seven workgroups per CU (4 x 64-1000: 128 8.8, 192 10.4, 256 10.6,
+    // 512 13.7; 24 x 100-2063: 256 24.1, 192 26.8, 512 27.8) and the reduction at
+    // some 48 partitions (one of 30,000: 1024 25.1, 512 26.7, 128 32.9; 2 x 6-7k
+    // GQA-4: 256 18.4, 128 20.2), twice that in fp32, whose rows are twice as
+    // long (one of 20,000: 128 39.4, 256 40.7, 512 47.2).  At most 3072 (64 x
+    // 16k-32k GQA-4 over four context draws: 75.4% of HBM peak against 73.8% for
+    // 2048, 75.1% for 2560, 74.3% for 3584 and 72.5% for 4096).
     const int64_t items = (int64_t)n_seqs * hkv;
-    if (items >= 1024 && cap <= 4096) {
+    const int64_t most_parts = elem_bytes == 4 ? 96 : 48;
+    if ((items >= 512 && cap <= 4096) || cap <= 2 * iter_tokens) {
       part = cap;
     } else {
-      part = 3072;
-      while (part > 256 && items * cdiv(cap, part) < 2048) part /= 2;
+      part = iter_tokens;
+      while (part < 3072 && (items * cdiv(cap, part) > 1792 || cdiv(cap, part) > most_parts)) part *= 2;
+      if (part > 3072) part = 3072;
     }
   }
   if (part > cap) part = cap;
@@ -528,6 +670,15 @@ static DecodePlan plan_decode(int32_t n_seqs, int32_t hq, int32_t hkv, int32_t b
   p.n_parts = (int32_t)cdiv(cap, part);
   p.ws_bytes = p.n_parts > 1 ? (size_t)n_seqs * hq * p.n_parts * (kHeadDim + 1) * sizeof(float) : 0;
   return p;
+}
+
+template <Dt DT, int G, int U, int NEW>
+static void launch_decode_p(const DecodeArgs& a, hipStream_t s) {
+  const dim3 grid(a.hkv, a.n_parts, a.n_seqs);
+  if (a.bs_shift >= 0)
+    hipLaunchKernelGGL((decode_paged_kernel<DT, G, U, true, NEW>), grid, dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((decode_paged_kernel<DT, G, U, false, NEW>), grid, dim3(256), 0, s, a);
 }
 
 template <Dt DT, int G>
@@ -539,13 +690,15 @@ static void launch_decode_t(const DecodeArgs& a, hipStream_t s) {
   // four (181) by 3% on 256 seqs x 1-2k at 64/8 heads (318.0 against
   // 328.2 us).
   constexpr int U = DT == Dt::FP32 ? 4 : 8;
-  dim3 grid(a.hkv, a.n_parts, a.n_seqs);
-  if (a.bs_shift >= 0)
-    hipLaunchKernelGGL((decode_paged_kernel<DT, G, U, true>), grid, dim3(256), 0, s, a);
-  else
-    hipLaunchKernelGGL((decode_paged_kernel<DT, G, U, false>), grid, dim3(256), 0, s, a);
+  if (a.qw) {
+    if constexpr (DT != Dt::FP32) launch_decode_p<DT, G, U, kQkv>(a, s);
+  } else if (a.k_new) {
+    launch_decode_p<DT, G, U, kAppend>(a, s);
+  } else {
+    launch_decode_p<DT, G, U, kNone>(a, s);
+  }
   if (a.n_parts > 1)
-    hipLaunchKernelGGL((decode_reduce_kernel<DT>), dim3(a.hq, a.n_seqs), dim3(64), 0, s, a);
+    hipLaunchKernelGGL((decode_reduce_kernel<DT>), dim3(a.hq, a.n_seqs), dim3(256), 0, s, a);
 }
 
 template <Dt DT>
@@ -571,10 +724,23 @@ extern "C" size_t aac_decode_workspace_bytes(int32_t n_seqs, int32_t n_q_heads, 
   (void)head_dim;
   if (n_seqs <= 0 || n_q_heads <= 0 || n_kv_heads <= 0 || block_size <= 0 || max_blocks_per_seq <= 0)
     return 0;
-  return plan_decode(n_seqs, n_q_heads, n_kv_heads, block_size, max_blocks_per_seq, max_context_len,
-                     partition_tokens)
-      .ws_bytes;
+  // the element type is not known here: the larger of the two plans
+  size_t most = 0;
+  for (int es : {2, 4})
+    most = std::max(most, plan_decode(n_seqs, n_q_heads, n_kv_heads, block_size, max_blocks_per_seq,
+                                      max_context_len, partition_tokens, es).ws_bytes);
+  return most;
 }
+
+// The new token of a step, when the launch appends it (DecodeArgs)
+struct NewToken {
+  const void *k = nullptr, *v = nullptr;
+  int64_t k_stride = 0, v_stride = 0;
+  const void *qw = nullptr, *kw = nullptr, *cos = nullptr, *sin = nullptr;
+  const int32_t* positions = nullptr;
+  int32_t max_pos = 0;
+  float eps = 0.f;
+};
 
 static int decode_common(const void* q, int64_t q_seq_stride, const void* k_cache,
                          const void* v_cache, int64_t num_blocks, int32_t block_size,
@@ -583,7 +749,7 @@ static int decode_common(const void* q, int64_t q_seq_stride, const void* k_cach
                          int32_t max_context_len, int32_t n_q_heads, int32_t n_kv_heads,
                          int32_t head_dim, float scale, void* out, int64_t out_seq_stride,
                          void* workspace, size_t workspace_bytes, int32_t partition_tokens,
-                         int32_t dtype, hipStream_t stream) {
+                         int32_t dtype, hipStream_t stream, const NewToken& nt = {}) {
   if (n_seqs < 0 || n_q_heads <= 0 || n_kv_heads <= 0 || num_blocks <= 0 || block_size <= 0 ||
       max_blocks_per_seq <= 0 || q_seq_stride < 0 || out_seq_stride < 0)
     return AAC_ERR_INVALID_ARGUMENT;
@@ -605,7 +771,7 @@ static int decode_common(const void* q, int64_t q_seq_stride, const void* k_cach
       (q_seq_stride * es) % 16 || (uintptr_t)out % 8 || (out_seq_stride * es) % 8)
     return AAC_ERR_MISALIGNED;
   const DecodePlan plan = plan_decode(n_seqs, n_q_heads, n_kv_heads, block_size,
-                                      max_blocks_per_seq, max_context_len, partition_tokens);
+                                      max_blocks_per_seq, max_context_len, partition_tokens, es);
   if (plan.ws_bytes) {
     if (!workspace || workspace_bytes < plan.ws_bytes) return AAC_ERR_WORKSPACE;
     if ((uintptr_t)workspace % 16) return AAC_ERR_MISALIGNED;
@@ -648,6 +814,17 @@ static int decode_common(const void* q, int64_t q_seq_stride, const void* k_cach
     a.ws_o = reinterpret_cast<float*>(workspace);
     a.ws_lse = a.ws_o + (size_t)n_seqs * n_q_heads * plan.n_parts * kHeadDim;
   }
+  a.k_new = nt.k;
+  a.v_new = nt.v;
+  a.k_new_stride = nt.k_stride;
+  a.v_new_stride = nt.v_stride;
+  a.qw = (const u16*)nt.qw;
+  a.kw = (const u16*)nt.kw;
+  a.cos = (const u16*)nt.cos;
+  a.sin = (const u16*)nt.sin;
+  a.positions = nt.positions;
+  a.max_pos = nt.max_pos;
+  a.eps = nt.eps;
   const int g = n_q_heads / n_kv_heads;
   int rc;
   switch (dt) {
@@ -739,6 +916,24 @@ extern "C" int aac_decode_append_paged(const void* q, int64_t q_seq_stride, cons
                                        size_t workspace_bytes, int32_t partition_tokens,
                                        int32_t dtype, void* stream) {
   if (head_dim != kHeadDim) return AAC_ERR_UNSUPPORTED;
+  // The append runs inside the attention launch when its rows suit the 16-byte
+  // loads there; anything else takes the general append first.
+  const int es = dtype == AAC_DTYPE_FP32 ? 4 : 2;
+  const int g = n_kv_heads > 0 && n_q_heads > 0 && n_q_heads % n_kv_heads == 0 ? n_q_heads / n_kv_heads : 0;
+  if (n_seqs > 0 && (g == 1 || g == 2 || g == 4 || g == 8) && k && v && k_cache && v_cache &&
+      block_tables && cache_seqlens && num_blocks > 0 && k_tok_stride >= (int64_t)n_kv_heads * head_dim &&
+      v_tok_stride >= (int64_t)n_kv_heads * head_dim && ((uintptr_t)k | (uintptr_t)v) % 16 == 0 &&
+      (k_tok_stride * es) % 16 == 0 && (v_tok_stride * es) % 16 == 0) {
+    NewToken nt;
+    nt.k = k;
+    nt.v = v;
+    nt.k_stride = k_tok_stride;
+    nt.v_stride = v_tok_stride;
+    return decode_common(q, q_seq_stride, k_cache, v_cache, num_blocks, block_size, block_tables,
+                         max_blocks_per_seq, cache_seqlens, 1, n_seqs, max_context_len, n_q_heads,
+                         n_kv_heads, head_dim, scale, out, out_seq_stride, workspace,
+                         workspace_bytes, partition_tokens, dtype, (hipStream_t)stream, nt);
+  }
   const int rc = aac_kv_append_paged(k, v, k_tok_stride, v_tok_stride, k_cache, v_cache, num_blocks,
                                      block_size, block_tables, max_blocks_per_seq, cache_seqlens,
                                      n_seqs, n_kv_heads, head_dim, dtype, stream);
@@ -747,4 +942,39 @@ extern "C" int aac_decode_append_paged(const void* q, int64_t q_seq_stride, cons
                        max_blocks_per_seq, cache_seqlens, 1, n_seqs, max_context_len, n_q_heads,
                        n_kv_heads, head_dim, scale, out, out_seq_stride, workspace,
                        workspace_bytes, partition_tokens, dtype, (hipStream_t)stream);
+}
+
+extern "C" int aac_decode_qkv_paged(
+    const void* qkv, int64_t qkv_row_stride, const void* q_norm_weight, const void* k_norm_weight,
+    float eps, const void* cos_table, const void* sin_table, int32_t max_position,
+    const int32_t* positions, void* k_cache, void* v_cache, int64_t num_blocks, int32_t block_size,
+    const int32_t* block_tables, int32_t max_blocks_per_seq, const int32_t* cache_seqlens,
+    int32_t n_seqs, int32_t max_context_len, int32_t n_q_heads, int32_t n_kv_heads,
+    int32_t head_dim, float scale, void* out, int64_t out_seq_stride, void* workspace,
+    size_t workspace_bytes, int32_t partition_tokens, int32_t dtype, void* stream) {
+  if (dtype != AAC_DTYPE_BF16 && dtype != AAC_DTYPE_FP16) return AAC_ERR_UNSUPPORTED;
+  if (head_dim != kHeadDim) return AAC_ERR_UNSUPPORTED;
+  if (n_seqs < 0 || n_q_heads <= 0 || n_kv_heads <= 0 || max_position <= 0) return AAC_ERR_INVALID_ARGUMENT;
+  if (qkv_row_stride < (int64_t)(n_q_heads + 2 * n_kv_heads) * head_dim) return AAC_ERR_SHAPE;
+  if (n_seqs == 0) return AAC_OK;
+  if (!qkv || !q_norm_weight || !k_norm_weight || !cos_table || !sin_table || !positions)
+    return AAC_ERR_INVALID_ARGUMENT;
+  if (((uintptr_t)qkv | (uintptr_t)q_norm_weight | (uintptr_t)k_norm_weight | (uintptr_t)cos_table |
+       (uintptr_t)sin_table) % 16 || qkv_row_stride % 8)
+    return AAC_ERR_MISALIGNED;
+  NewToken nt;
+  nt.k = (const u16*)qkv + (int64_t)n_q_heads * kHeadDim;
+  nt.v = (const u16*)qkv + (int64_t)(n_q_heads + n_kv_heads) * kHeadDim;
+  nt.k_stride = nt.v_stride = qkv_row_stride;
+  nt.qw = q_norm_weight;
+  nt.kw = k_norm_weight;
+  nt.cos = cos_table;
+  nt.sin = sin_table;
+  nt.positions = positions;
+  nt.max_pos = max_position;
+  nt.eps = eps;
+  return decode_common(qkv, qkv_row_stride, k_cache, v_cache, num_blocks, block_size, block_tables,
+                       max_blocks_per_seq, cache_seqlens, 1, n_seqs, max_context_len, n_q_heads,
+                       n_kv_heads, head_dim, scale, out, out_seq_stride, workspace,
+                       workspace_bytes, partition_tokens, dtype, (hipStream_t)stream, nt);
 }

@@ -115,35 +115,27 @@ __device__ __forceinline__ int64_t cache_row(const QkArgs& a, int64_t t) {
   return crow;
 }
 
-// One head row of token t, held by the 16 lanes of a DPP row (lane li owns
-// dims [8li, 8li+8)): a value head is copied into the cache; a query or key
-// head gets RMSNorm over the head (model/model.py:47-52) and RoPE, out =
+// One query or key head row, held by the 16 lanes of a DPP row (lane li owns
+// dims [8li, 8li+8)): RMSNorm over the head (model/model.py:47-52) and RoPE, out =
 // x*cos + rotate_half(x)*sin with each product and the sum rounded
 // (model/model.py:90-99); rotate_half pairs dim d with d +- 64, i.e. lane li
 // with lane li ^ 8 (DPP row_ror:8).  The caller keeps the row's 16 lanes
-// together on every branch.
-// sf holds sin with the sign of rotate_half folded in: negative in the lanes
-// of the first half (li < 8), see signed_sin.
-template <Dt DT, bool NT = false>
-__device__ __forceinline__ void norm_rope_head(const QkArgs& a, int64_t t, int hh, int li,
-                                               const u32x4& xr, int64_t crow, const float* wf,
-                                               const float* cf, const float* sf) {
+// together on every branch.  sf holds sin with the sign of rotate_half folded
+// in: negative in the lanes of the first half (li < 8), see signed_sin.
+template <Dt DT>
+__device__ __forceinline__ u32x4 norm_rope_row(const u32x4& xr, float eps, const float* wf, const float* cf,
+                                               const float* sf) {
   // Each product and the sum are rounded separately; for fp16 those rounds
   // become half-precision operations, which contraction would merge into one
   // fused multiply-add (a single rounding, unlike the torch expression).
 #pragma clang fp contract(off)
-  if (hh >= a.hq + a.hkv) {  // value head
-    if (crow >= 0)
-      put16<NT>(a.v_cache + (crow * a.hkv + (hh - a.hq - a.hkv)) * kHeadDimFused + li * 8, xr);
-    return;
-  }
   float x[8];
   unpack8<DT>(xr, x);
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) ss = fmaf(x[i], x[i], ss);
   ss = row16_sum(ss);
-  const float rs = __frsqrt_rn(ss / (float)kHeadDimFused + a.eps);
+  const float rs = __frsqrt_rn(ss / (float)kHeadDimFused + eps);
 #pragma unroll
   for (int i = 0; i < 8; ++i) x[i] *= rs;
 #pragma unroll
@@ -167,6 +159,21 @@ __device__ __forceinline__ void norm_rope_head(const QkArgs& a, int64_t t, int h
     round2<DT>(r[0], r[1]);
     packed[i / 2] = Cvt<DT>::pack(c[0] + r[0], c[1] + r[1]);
   }
+  return packed;
+}
+
+// One head row of token t: a value head is copied into the cache, a query or
+// key head goes through norm_rope_row.
+template <Dt DT, bool NT = false>
+__device__ __forceinline__ void norm_rope_head(const QkArgs& a, int64_t t, int hh, int li,
+                                               const u32x4& xr, int64_t crow, const float* wf,
+                                               const float* cf, const float* sf) {
+  if (hh >= a.hq + a.hkv) {  // value head
+    if (crow >= 0)
+      put16<NT>(a.v_cache + (crow * a.hkv + (hh - a.hq - a.hkv)) * kHeadDimFused + li * 8, xr);
+    return;
+  }
+  const u32x4 packed = norm_rope_row<DT>(xr, a.eps, wf, cf, sf);
   if (hh < a.hq) {
     put16<NT>(a.q_out + (t * a.hq + hh) * kHeadDimFused + li * 8, packed);
   } else {

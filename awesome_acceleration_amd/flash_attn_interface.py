@@ -40,6 +40,7 @@ __all__ = [
     "flash_attn_with_kvcache",
     "flash_attn_func",
     "decode_paged",
+    "decode_qkv_paged",
 ]
 
 _CHECK = os.environ.get("AAC_CHECK", "0") not in ("", "0")
@@ -338,6 +339,49 @@ def decode_paged(q, k_cache, v_cache, block_tables, context_lens, softmax_scale=
         ws.data_ptr() if ws is not None else None, ws_bytes, int(partition_tokens),
         _dtype_code(q), _stream(q))
     _lib.check(rc, "aac_decode_paged")
+    return out
+
+
+def decode_qkv_paged(qkv, n_q_heads, q_norm_weight, k_norm_weight, eps, cos, sin, positions,
+                     k_cache, v_cache, block_tables, cache_seqlens, softmax_scale=None,
+                     max_context_len=None):
+    """One decode step's attention from the rows of the fused QKV projection,
+    ``qkv [B, (Hq + 2 Hkv) * D]``: q/k RMSNorm + RoPE at ``positions``, the
+    append at ``cache_seqlens`` and the attention over ``cache_seqlens + 1``
+    tokens (model/model.py:219-240) in one launch (and the reduction of a
+    split).  Returns ``[B, Hq, D]``; bf16 and fp16."""
+    _on_gpu(qkv, q_norm_weight, k_norm_weight, cos, sin, positions, k_cache, v_cache, block_tables,
+            cache_seqlens)
+    _require(qkv.dim() == 2 and qkv.stride(1) == 1, "qkv must be [B, width]")
+    B = qkv.shape[0]
+    _require(k_cache.dim() == 4 and k_cache.shape == v_cache.shape and k_cache.is_contiguous()
+             and v_cache.is_contiguous(), "caches must be contiguous [num_blocks, block, Hkv, D], alike")
+    nblk, bs, hkv, D = k_cache.shape
+    _require(qkv.shape[1] == (n_q_heads + 2 * hkv) * D, "qkv width")
+    _require(n_q_heads % hkv == 0, "query heads must be a multiple of KV heads")
+    for t in (k_cache, v_cache, q_norm_weight, k_norm_weight, cos, sin):
+        _require(t.dtype == qkv.dtype and t.is_contiguous(), "one dtype, contiguous weights and tables")
+    _require(q_norm_weight.shape == (D,) and k_norm_weight.shape == (D,), "norm weights must be [D]")
+    _require(cos.dim() == 2 and cos.shape[1] == D and sin.shape == cos.shape, "cos/sin must be [P, D]")
+    for t in (positions, cache_seqlens):
+        _require(t.dtype == torch.int32 and t.shape == (B,) and t.is_contiguous(),
+                 "positions and cache_seqlens must be contiguous int32 [B]")
+    _require(block_tables.dtype == torch.int32 and block_tables.dim() == 2
+             and block_tables.shape[0] == B and block_tables.is_contiguous(),
+             "block_tables must be contiguous int32 [B, max_blocks]")
+    out = torch.empty((B, n_q_heads, D), dtype=qkv.dtype, device=qkv.device)
+    mb, mcl = block_tables.shape[1], int(max_context_len or 0)
+    L = _lib.lib()
+    ws_bytes = L.aac_decode_workspace_bytes(B, n_q_heads, hkv, D, bs, mb, mcl, 0)
+    ws = _workspace(ws_bytes, qkv.device) if ws_bytes else None
+    rc = L.aac_decode_qkv_paged(
+        qkv.data_ptr(), qkv.stride(0), q_norm_weight.data_ptr(), k_norm_weight.data_ptr(),
+        float(eps), cos.data_ptr(), sin.data_ptr(), cos.shape[0], positions.data_ptr(),
+        k_cache.data_ptr(), v_cache.data_ptr(), nblk, bs, block_tables.data_ptr(), mb,
+        cache_seqlens.data_ptr(), B, mcl, n_q_heads, hkv, D, _scale(softmax_scale, D),
+        out.data_ptr(), n_q_heads * D, ws.data_ptr() if ws is not None else None, ws_bytes, 0,
+        _dtype_code(qkv), _stream(qkv))
+    _lib.check(rc, "aac_decode_qkv_paged")
     return out
 
 

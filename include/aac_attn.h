@@ -237,6 +237,8 @@ int aac_decode_paged_noalloc(const void* q, int64_t q_seq_stride, const void* k_
  * cache_seqlens[b] (aac_kv_append_paged), then attend over
  * cache_seqlens[b] + 1 tokens.  cache_seqlens is not modified.
  * max_context_len bounds cache_seqlens[b] + 1 (<= 0: table capacity).
+ * The append runs inside the attention launch: as in flash_attn, sequences of
+ * one call do not see each other's new tokens in a shared block.
  * Replaces model/model.py:233-240.
  */
 int aac_decode_append_paged(const void* q, int64_t q_seq_stride, const void* k, const void* v,
@@ -248,6 +250,25 @@ int aac_decode_append_paged(const void* q, int64_t q_seq_stride, const void* k, 
                             void* out, int64_t out_seq_stride, void* workspace,
                             size_t workspace_bytes, int32_t partition_tokens, int32_t dtype,
                             void* stream);
+
+/*
+ * The same step from the rows of the fused QKV projection, qkv
+ * [n_seqs, (n_q_heads + 2 n_kv_heads) * head_dim]: q/k RMSNorm + RoPE at
+ * positions[b] (model/model.py:219-228, as aac_qk_norm_rope_store), the append
+ * of k and v at cache_seqlens[b], and the attention over cache_seqlens[b] + 1
+ * tokens (model/model.py:233-240), without the normalised q and k in memory.
+ * dtype bf16 or fp16; the workspace is aac_decode_workspace_bytes'.
+ */
+int aac_decode_qkv_paged(const void* qkv, int64_t qkv_row_stride, const void* q_norm_weight,
+                         const void* k_norm_weight, float eps, const void* cos_table,
+                         const void* sin_table, int32_t max_position, const int32_t* positions,
+                         void* k_cache, void* v_cache, int64_t num_blocks, int32_t block_size,
+                         const int32_t* block_tables, int32_t max_blocks_per_seq,
+                         const int32_t* cache_seqlens, int32_t n_seqs, int32_t max_context_len,
+                         int32_t n_q_heads, int32_t n_kv_heads, int32_t head_dim, float scale,
+                         void* out, int64_t out_seq_stride, void* workspace,
+                         size_t workspace_bytes, int32_t partition_tokens, int32_t dtype,
+                         void* stream);
 
 /* ------------------------------------------------------------------------
  * Fused kernels of the attention call site.  Each replaces a chain of small

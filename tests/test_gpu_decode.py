@@ -15,6 +15,7 @@ import torch
 
 import oracle
 from awesome_acceleration_amd import flash_attn_interface as fai
+from awesome_acceleration_amd import fused as fz
 from cases import config1_inputs, sha256, tiny_decode_inputs
 from gpu_util import bf16_np_to_f64, bytes_of, check_attention, f64, np_of, t_of
 
@@ -371,3 +372,83 @@ def test_decode_constant_values_return_that_value(gpu, dtype, hq, hkv, part):
     bad = err > ulp * want.abs()
     assert not bad.any(), f"{int(bad.sum())} values beyond one ulp (max err {float(err.max()):.3e})"
     print(f"  exact: {bool((err == 0).all())}, max err {float(err.max()):.3e}", flush=True)
+
+
+def _append_case(gpu, dtype, hq, hkv, bs, seed):
+    """Caches, tables and positions whose new token falls on the ends of blocks,
+    partitions and the table, and three sequences without an append: position
+    -1, one past the table, a block number outside the cache."""
+    g = torch.Generator(device=gpu).manual_seed(seed)
+    W = 7
+    lens = [0, 1, bs - 1, bs, 127, 128, 255, 256, 3 * bs - 1, W * bs - 1, -1, W * bs, 2 * bs + 3]
+    lens = [min(x, W * bs) for x in lens]
+    B = len(lens)
+    pool = B * W + 3
+    kc = torch.randn((pool, bs, hkv, 128), generator=g, device=gpu).to(dtype)
+    vc = torch.randn((pool, bs, hkv, 128), generator=g, device=gpu).to(dtype)
+    bt = torch.randperm(pool, generator=g, device=gpu)[:B * W].view(B, W).to(torch.int32)
+    bt[-1, 2] = pool + 5  # the block of the last sequence's new token
+    slots = [int(bt[b, p // bs]) * bs + p % bs
+             if 0 <= p < W * bs and int(bt[b, p // bs]) < pool else -1 for b, p in enumerate(lens)]
+    for b, s in enumerate(slots):  # a row not yet written may hold anything
+        if s >= 0:
+            vc.view(-1, hkv, 128)[s] = float("nan")
+    return g, kc, vc, bt, torch.tensor(lens, dtype=torch.int32, device=gpu), slots
+
+
+def _close_decode(out, ref, dtype, vmax):
+    """Two correct results of one call differ by at most twice the bound of
+    check_attention: the rounding of the output and of the probabilities
+    (sum p |v| <= max |v|); fp32: the sums' rounding."""
+    eps = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -19}[dtype]
+    err = (out.float() - ref.float()).abs()
+    assert torch.isfinite(out.float()).all()
+    assert (err <= 2 * eps * (ref.float().abs() + vmax)).all(), float(err.max())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("hq,hkv,bs", [(16, 8, 64), (32, 8, 100), (8, 8, 16), (16, 2, 64)])
+def test_append_inside_the_attention_launch(gpu, dtype, hq, hkv, bs):
+    """The append in the attention launch leaves the caches as a store before it
+    would, bit for bit, and attends the new token (whose key is made to weigh)."""
+    print(f"case: append in launch {dtype} {hq}/{hkv} block {bs}", flush=True)
+    g, kc, vc, bt, sl, slots = _append_case(gpu, dtype, hq, hkv, bs, 12)
+    B = len(slots)
+    q = torch.randn((B, 1, hq, 128), generator=g, device=gpu).to(dtype)
+    wide = torch.randn((B, 3, hkv, 128), generator=g, device=gpu).to(dtype)
+    wide[:, 0] += (0.3 * q[:, 0, ::hq // hkv].float()).to(dtype)
+    k, v = wide[:, :1], wide[:, 1:2]  # strided rows
+    kc2, vc2 = kc.clone(), vc.clone()
+    for b, s in enumerate(slots):
+        if s >= 0:
+            kc2.view(-1, hkv, 128)[s], vc2.view(-1, hkv, 128)[s] = k[b, 0], v[b, 0]
+    for splits in (0, 3):
+        out = fai.flash_attn_with_kvcache(q, kc, vc, k=k, v=v, cache_seqlens=sl, block_table=bt,
+                                          num_splits=splits)
+        ref = fai.flash_attn_with_kvcache(q, kc2, vc2, cache_seqlens=sl + 1, block_table=bt,
+                                          num_splits=splits)
+        torch.cuda.synchronize()
+        _close_decode(out, ref, dtype, float(vc2.float().abs().max()))
+        assert torch.equal(kc, kc2) and torch.equal(vc, vc2)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,bs", [(16, 8, 64), (32, 8, 100), (8, 8, 16), (16, 2, 64)])
+def test_decode_from_projection_rows(gpu, dtype, hq, hkv, bs):
+    """decode_qkv_paged = q/k norm + RoPE + append, then decode: the caches bit
+    for bit, the output within the rounding bound."""
+    print(f"case: decode from qkv rows {dtype} {hq}/{hkv} block {bs}", flush=True)
+    g, kc, vc, bt, sl, slots = _append_case(gpu, dtype, hq, hkv, bs, 13)
+    B = len(slots)
+    qkv = torch.randn((B, (hq + 2 * hkv) * 128), generator=g, device=gpu).to(dtype)
+    qw, kw = (1 + 0.3 * torch.randn((2, 128), generator=g, device=gpu)).to(dtype)
+    ang = torch.rand((300, 128), generator=g, device=gpu) * 6.28
+    cos, sin = ang.cos().to(dtype), ang.sin().to(dtype)  # positions past 299 clamp in both
+    kc2, vc2 = kc.clone(), vc.clone()
+    q, _ = fz.qk_norm_rope_store(qkv, hq, hkv, qw, kw, 1e-6, cos, sin, sl, kc2, vc2,
+                                 block_tables=bt, cache_seqlens=sl, want_k=False)
+    ref = fai.decode_paged(q, kc2, vc2, bt, sl + 1)
+    out = fai.decode_qkv_paged(qkv, hq, qw, kw, 1e-6, cos, sin, sl, kc, vc, bt, sl)
+    torch.cuda.synchronize()
+    assert torch.equal(kc, kc2) and torch.equal(vc, vc2)
+    _close_decode(out, ref, dtype, float(vc2.float().abs().max()))
