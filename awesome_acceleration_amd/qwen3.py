@@ -40,6 +40,7 @@ __all__ = ["Qwen3Config", "Qwen3ForCausalLM", "PagedKVCache", "StepMeta"]
 
 
 NORM_GEMM_ROWS = 16
+LM_HEAD_ROWS = 8
 
 
 @dataclass
@@ -271,11 +272,22 @@ class Qwen3ForCausalLM:
         lin = fz.linear if small else F.linear
         merged = small and T <= self.norm_gemm_rows
         for li, L in enumerate(self.layers):
-            if delta is None:
+            if merged:
+                # norm + projection, then q/k norm + RoPE, KV append and attention
+                qkv, r = fz.rmsnorm_linear(res if delta is None else delta, L["ln1"], eps, L["qkv"],
+                                           residual=None if delta is None else res)
+                res = res if delta is None else r
+                attn = fai.decode_qkv_paged(
+                    qkv, self.hq, L["q_norm"], L["k_norm"], eps, self.rope.cos, self.rope.sin, pos,
+                    cache.k(li), cache.v(li), meta.block_tables, meta.cache_seqlens,
+                    softmax_scale=self.scale, max_context_len=meta.max_context_len)
+            elif delta is None:
                 x = fz.rmsnorm(res, L["ln1"], eps)
             else:
                 x, res = fz.rmsnorm(delta, L["ln1"], eps, residual=res)
-            if small:  # projection, q/k norm + RoPE and the KV append in one launch
+            if merged:
+                pass
+            elif small:  # projection, q/k norm + RoPE and the KV append in one launch
                 q, _ = fz.qkv_norm_rope_store(
                     x, L["qkv"], self.hq, self.hkv, L["q_norm"], L["k_norm"], eps, self.rope.cos,
                     self.rope.sin, pos, cache.k(li), cache.v(li), block_tables=meta.block_tables,
@@ -296,7 +308,7 @@ class Qwen3ForCausalLM:
                         self.rope.sin, pos, cache.k(li), cache.v(li),
                         block_tables=meta.block_tables, cache_seqlens=meta.cache_seqlens,
                         want_k=False)
-            if not prefill:
+            if not prefill and not merged:
                 attn = fai.decode_paged(q, cache.k(li), cache.v(li), meta.block_tables,
                                         meta.context_lens, softmax_scale=self.scale,
                                         max_context_len=meta.max_context_len)
@@ -313,7 +325,12 @@ class Qwen3ForCausalLM:
         if prefill:
             delta, res = delta[meta.last_idx], res[meta.last_idx]
         h, _ = fz.rmsnorm(delta, self.norm, eps, residual=res)
-        return F.linear(h, self.embed)  # tied embeddings
+        # tied embeddings; up to LM_HEAD_ROWS rows the streaming kernel of the
+        # few-row projections (hidden 1024, vocabulary 151,936, us against the
+        # library: 1-4 rows 46.0 / 53, 8 48.6 / 54, 16 64.2 / 55)
+        if merged and T <= LM_HEAD_ROWS and self.embed.shape[0] % 32 == 0:
+            return fz.linear(h, self.embed)
+        return F.linear(h, self.embed)
 
     @torch.no_grad()
     def forward(self, input_ids: torch.Tensor, meta: StepMeta, cache: PagedKVCache,
