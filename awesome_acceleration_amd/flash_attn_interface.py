@@ -24,6 +24,7 @@ itself, model/model.py:241).
 """
 from __future__ import annotations
 
+import functools
 import math
 import os
 import threading
@@ -46,8 +47,14 @@ __all__ = [
 _CHECK = os.environ.get("AAC_CHECK", "0") not in ("", "0")
 
 
+# The current stream's handle by device index, without the Stream object that
+# torch.cuda.current_stream builds (0.1 us against 1.4).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+    lambda index: torch.cuda.current_stream(index).cuda_stream)
+
+
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.get_device())
 
 
 def _require(cond: bool, msg: str) -> None:
@@ -61,24 +68,29 @@ def _dtype_code(t: torch.Tensor) -> int:
     return code
 
 
-def _on_gpu(*ts: Optional[torch.Tensor]) -> torch.device:
-    dev = None
+def _on_gpu(*ts: Optional[torch.Tensor]) -> None:
+    dev = -1
     for t in ts:
         if t is None:
             continue
-        _require(t.is_cuda, "all tensors must be on a GPU (no CPU path exists)")
-        if dev is None:
-            dev = t.device
-        _require(t.device == dev, "all tensors must be on the same GPU")
-    return dev
+        d = t.get_device()  # -1: not on a GPU
+        if d < 0:
+            raise RuntimeError("all tensors must be on a GPU (no CPU path exists)")
+        if d != dev:
+            if dev >= 0:
+                raise RuntimeError("all tensors must be on the same GPU")
+            dev = d
 
 
 def _token_rows(t: torch.Tensor, name: str) -> int:
     """Token stride (elements) of a [N, H, D] tensor whose [H, D] block is contiguous."""
-    _require(t.dim() == 3, f"{name} must be [tokens, heads, head_dim]")
-    _require(t.stride(2) == 1 and t.stride(1) == t.shape[2],
-             f"{name}: heads and head_dim must be contiguous within a token")
-    return t.stride(0) if t.shape[0] > 1 else t.shape[1] * t.shape[2]
+    shape = t.shape
+    if len(shape) != 3:
+        raise RuntimeError(f"{name} must be [tokens, heads, head_dim]")
+    st = t.stride()
+    if st[2] != 1 or st[1] != shape[2]:
+        raise RuntimeError(f"{name}: heads and head_dim must be contiguous within a token")
+    return st[0] if shape[0] > 1 else shape[1] * shape[2]
 
 
 # ---------------------------------------------------------------- workspace
@@ -90,7 +102,13 @@ _ws_retired: list[torch.Tensor] = []
 
 def _stream_key(device: torch.device) -> tuple[int, int]:
     idx = device.index if device.index is not None else torch.cuda.current_device()
-    return idx, torch.cuda.current_stream(idx).cuda_stream
+    return idx, _raw_stream(idx)
+
+
+@functools.lru_cache(maxsize=4096)
+def _decode_ws_bytes(*args: int) -> int:
+    """aac_decode_workspace_bytes: host arithmetic on its integer arguments."""
+    return _lib.lib().aac_decode_workspace_bytes(*args)
 
 
 def _workspace(nbytes: int, device: torch.device) -> torch.Tensor:
@@ -209,17 +227,27 @@ def _unsupported(dropout_p, window_size, softcap, alibi_slopes, return_attn_prob
 
 
 def _prefill_checks(q, k, v, cu_seqlens_q, cu_seqlens_k):
+    """Token strides of q, k, v, all arguments checked (one condition per line of
+    the common case: a call's host time is its latency for a short prompt)."""
     _on_gpu(q, k, v, cu_seqlens_q, cu_seqlens_k)
     qs, ks, vs = _token_rows(q, "q"), _token_rows(k, "k"), _token_rows(v, "v")
-    _require(q.dtype in (torch.bfloat16, torch.float16), "prefill supports fp16 and bf16 only")
-    _require(q.dtype == k.dtype == v.dtype, "q, k, v must share a dtype")
-    _require(k.shape == v.shape, "k and v must have the same shape")
-    _require(q.shape[2] == k.shape[2], "head_dim mismatch")
-    _require(q.shape[1] % k.shape[1] == 0, "number of query heads must be a multiple of KV heads")
-    for c in (cu_seqlens_q, cu_seqlens_k):
-        _require(c.dtype == torch.int32 and c.dim() == 1 and c.is_contiguous(),
-                 "cu_seqlens must be contiguous int32 [batch+1]")
-    _require(cu_seqlens_q.shape == cu_seqlens_k.shape, "cu_seqlens_q / cu_seqlens_k length mismatch")
+    dt = q.dtype
+    if dt is not torch.bfloat16 and dt is not torch.float16:
+        raise RuntimeError("prefill supports fp16 and bf16 only")
+    if k.dtype is not dt or v.dtype is not dt:
+        raise RuntimeError("q, k, v must share a dtype")
+    kshape, qshape = k.shape, q.shape
+    if kshape != v.shape:
+        raise RuntimeError("k and v must have the same shape")
+    if qshape[2] != kshape[2]:
+        raise RuntimeError("head_dim mismatch")
+    if qshape[1] % kshape[1]:
+        raise RuntimeError("number of query heads must be a multiple of KV heads")
+    for c in (cu_seqlens_q,) if cu_seqlens_q is cu_seqlens_k else (cu_seqlens_q, cu_seqlens_k):
+        if c.dtype is not torch.int32 or c.dim() != 1 or not c.is_contiguous():
+            raise RuntimeError("cu_seqlens must be contiguous int32 [batch+1]")
+    if cu_seqlens_q is not cu_seqlens_k and cu_seqlens_q.shape != cu_seqlens_k.shape:
+        raise RuntimeError("cu_seqlens_q / cu_seqlens_k length mismatch")
     return qs, ks, vs
 
 
@@ -267,15 +295,20 @@ def varlen_prefill_with_kvcache(q, k, v, cu_seqlens, max_seqlen, k_cache, v_cach
     attention, in one call (the per-layer block llm.py:171-184)."""
     qs, ks, vs = _prefill_checks(q, k, v, cu_seqlens, cu_seqlens)
     _on_gpu(q, k_cache, v_cache, slot_mapping)
-    _require(k_cache.dtype == v_cache.dtype == q.dtype, "cache dtype mismatch")
-    _require(k_cache.is_contiguous() and v_cache.is_contiguous(), "caches must be contiguous")
-    _require(k_cache.shape == v_cache.shape, "k_cache and v_cache must have the same shape")
-    _require(tuple(k_cache.shape[-2:]) == tuple(k.shape[1:]), "cache row shape != [Hkv, D]")
-    _require(slot_mapping.dtype == torch.int64 and slot_mapping.dim() == 1
-             and slot_mapping.shape[0] == k.shape[0] and slot_mapping.is_contiguous(),
-             "slot_mapping must be contiguous int64 [N]")
+    if k_cache.dtype is not q.dtype or v_cache.dtype is not q.dtype:
+        raise RuntimeError("cache dtype mismatch")
+    if not (k_cache.is_contiguous() and v_cache.is_contiguous()):
+        raise RuntimeError("caches must be contiguous")
+    if k_cache.shape != v_cache.shape:
+        raise RuntimeError("k_cache and v_cache must have the same shape")
+    if k_cache.shape[-2:] != k.shape[1:]:
+        raise RuntimeError("cache row shape != [Hkv, D]")
+    if (slot_mapping.dtype is not torch.int64 or slot_mapping.dim() != 1
+            or slot_mapping.shape[0] != k.shape[0] or not slot_mapping.is_contiguous()):
+        raise RuntimeError("slot_mapping must be contiguous int64 [N]")
     rows = k_cache.numel() // (k.shape[1] * k.shape[2])
-    _check_slots(slot_mapping, rows)
+    if _CHECK:
+        _check_slots(slot_mapping, rows)
     scale = q.shape[-1] ** -0.5 if softmax_scale is None else float(softmax_scale)
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     rc = _lib.lib().aac_prefill_varlen_store(
@@ -330,7 +363,7 @@ def decode_paged(q, k_cache, v_cache, block_tables, context_lens, softmax_scale=
     mb = block_tables.shape[1]
     mcl = int(max_context_len or 0)
     L = _lib.lib()
-    ws_bytes = L.aac_decode_workspace_bytes(B, Hq, hkv, D, bs, mb, mcl, int(partition_tokens))
+    ws_bytes = _decode_ws_bytes(B, Hq, hkv, D, bs, mb, mcl, int(partition_tokens))
     ws = _workspace(ws_bytes, q.device) if ws_bytes else None
     rc = L.aac_decode_paged(
         q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(), nblk, bs,
@@ -372,7 +405,7 @@ def decode_qkv_paged(qkv, n_q_heads, q_norm_weight, k_norm_weight, eps, cos, sin
     out = torch.empty((B, n_q_heads, D), dtype=qkv.dtype, device=qkv.device)
     mb, mcl = block_tables.shape[1], int(max_context_len or 0)
     L = _lib.lib()
-    ws_bytes = L.aac_decode_workspace_bytes(B, n_q_heads, hkv, D, bs, mb, mcl, 0)
+    ws_bytes = _decode_ws_bytes(B, n_q_heads, hkv, D, bs, mb, mcl, 0)
     ws = _workspace(ws_bytes, qkv.device) if ws_bytes else None
     rc = L.aac_decode_qkv_paged(
         qkv.data_ptr(), qkv.stride(0), q_norm_weight.data_ptr(), k_norm_weight.data_ptr(),
@@ -390,12 +423,18 @@ def _scale(softmax_scale, D):
 
 
 def _check_cache(q, k_cache, v_cache):
-    _require(k_cache.dim() == 4 and k_cache.shape == v_cache.shape,
-             "caches must be [num_blocks, block_size, Hkv, D] with equal shapes")
-    _require(k_cache.is_contiguous() and v_cache.is_contiguous(), "caches must be contiguous")
-    _require(k_cache.dtype == v_cache.dtype == q.dtype, "q and caches must share a dtype")
-    _require(k_cache.shape[3] == q.shape[-1], "head_dim mismatch")
-    _require(q.shape[-2] % k_cache.shape[2] == 0, "query heads must be a multiple of KV heads")
+    shape, dt = k_cache.shape, q.dtype
+    if len(shape) != 4 or shape != v_cache.shape:
+        raise RuntimeError("caches must be [num_blocks, block_size, Hkv, D] with equal shapes")
+    if not (k_cache.is_contiguous() and v_cache.is_contiguous()):
+        raise RuntimeError("caches must be contiguous")
+    if k_cache.dtype is not dt or v_cache.dtype is not dt:
+        raise RuntimeError("q and caches must share a dtype")
+    qshape = q.shape
+    if shape[3] != qshape[-1]:
+        raise RuntimeError("head_dim mismatch")
+    if qshape[-2] % shape[2]:
+        raise RuntimeError("query heads must be a multiple of KV heads")
 
 
 def flash_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, rotary_cos=None, rotary_sin=None,
@@ -416,71 +455,86 @@ def flash_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, rotary_cos=None
     ``cache_seqlens[b]``.  ``cache_seqlens`` is not modified.  Returns a new
     ``[B, 1, Hq, D]`` tensor.
     """
-    _unsupported(0.0, window_size, softcap, alibi_slopes, False)
+    if softcap or alibi_slopes is not None or window_size != (-1, -1):
+        _unsupported(0.0, window_size, softcap, alibi_slopes, False)
     if rotary_cos is not None or rotary_sin is not None:
         raise NotImplementedError("rotary inside the kernel is not supported; apply RoPE first")
     if cache_leftpad is not None:
         raise NotImplementedError("cache_leftpad is not supported")
     if return_softmax_lse:
         raise NotImplementedError("return_softmax_lse is not supported")
-    _require(q.dim() == 4, "q must be [B, S, Hq, D]")
+    if q.dim() != 4:
+        raise RuntimeError("q must be [B, S, Hq, D]")
     B, S, Hq, D = q.shape
     if S != 1:
         raise NotImplementedError("only one query token per sequence (decode) is supported")
-    _require((k is None) == (v is None), "k and v must be given together")
+    if (k is None) != (v is None):
+        raise RuntimeError("k and v must be given together")
     _on_gpu(q, k_cache, v_cache, k, v, cache_batch_idx, block_table)
     _check_cache(q, k_cache, v_cache)
-    dev = q.device
+    nblk, bs, hkv, _ = k_cache.shape
     if block_table is None:
         if cache_batch_idx is None:
-            tables = torch.arange(B, dtype=torch.int32, device=dev).view(B, 1)
+            tables = torch.arange(B, dtype=torch.int32, device=q.device)
         else:
             tables = cache_batch_idx.to(torch.int32).reshape(B, 1).contiguous()
+        mb = 1
     else:
-        _require(cache_batch_idx is None, "cache_batch_idx cannot be combined with block_table")
-        _require(block_table.dtype == torch.int32 and block_table.dim() == 2
-                 and block_table.shape[0] == B, "block_table must be int32 [B, max_blocks]")
+        if cache_batch_idx is not None:
+            raise RuntimeError("cache_batch_idx cannot be combined with block_table")
+        if block_table.dtype is not torch.int32 or block_table.dim() != 2 or block_table.shape[0] != B:
+            raise RuntimeError("block_table must be int32 [B, max_blocks]")
         tables = block_table.contiguous()
+        mb = block_table.shape[1]
     if cache_seqlens is None:
         raise RuntimeError("cache_seqlens is required")
     if isinstance(cache_seqlens, int):
-        seqlens = torch.full((B,), cache_seqlens, dtype=torch.int32, device=dev)
+        seqlens = torch.full((B,), cache_seqlens, dtype=torch.int32, device=q.device)
     else:
         _on_gpu(q, cache_seqlens)
         seqlens = cache_seqlens.to(torch.int32).contiguous()
-        _require(seqlens.shape == (B,), "cache_seqlens must be [B]")
-    nblk, bs, hkv = k_cache.shape[0], k_cache.shape[1], k_cache.shape[2]
-    mb = tables.shape[1]
-    q3 = q.view(B, Hq, D) if q.is_contiguous() else q.reshape(B, Hq, D)
-    _require(q3.stride(2) == 1 and q3.stride(1) == D, "q heads/head_dim must be contiguous")
-    out = torch.empty((B, 1, Hq, D), dtype=q.dtype, device=dev)
+        if seqlens.shape != (B,):
+            raise RuntimeError("cache_seqlens must be [B]")
+    q3 = q if q.is_contiguous() else q.reshape(B, Hq, D)
+    if q3 is q:
+        q_stride = Hq * D
+    else:
+        q_stride = q3.stride(0)
+        if q3.stride(2) != 1 or q3.stride(1) != D:
+            raise RuntimeError("q heads/head_dim must be contiguous")
+    out = torch.empty((B, 1, Hq, D), dtype=q.dtype, device=q.device)
     mcl = int(max_context_len or 0)
     part = 0
     if num_splits and num_splits > 0:
         cap = min(mcl, mb * bs) if mcl > 0 else mb * bs
         part = max(1, math.ceil(cap / int(num_splits)))
     L = _lib.lib()
-    ws_bytes = L.aac_decode_workspace_bytes(B, Hq, hkv, D, bs, mb, mcl, part)
-    ws = _workspace(ws_bytes, dev) if ws_bytes else None
-    wsp = ws.data_ptr() if ws is not None else None
+    ws_bytes = _decode_ws_bytes(B, Hq, hkv, D, bs, mb, mcl, part)
+    wsp = _workspace(ws_bytes, q.device).data_ptr() if ws_bytes else None
     if k is None:
         rc = L.aac_decode_paged(
-            q3.data_ptr(), q3.stride(0), k_cache.data_ptr(), v_cache.data_ptr(), nblk, bs,
+            q3.data_ptr(), q_stride, k_cache.data_ptr(), v_cache.data_ptr(), nblk, bs,
             tables.data_ptr(), mb, seqlens.data_ptr(), B, mcl, Hq, hkv, D, _scale(softmax_scale, D),
             out.data_ptr(), Hq * D, wsp, ws_bytes, part, _dtype_code(q), _stream(q))
         _lib.check(rc, "aac_decode_paged")
         return out
-    _require(k.shape == v.shape and k.shape[0] == B and k.shape[1] == 1,
-             "k/v must be [B, 1, Hkv, D]")
-    _require(k.dtype == q.dtype and v.dtype == q.dtype, "k/v dtype mismatch")
-    k3 = k.reshape(B, k.shape[2], D) if not (k.stride(3) == 1 and k.stride(2) == D) else \
-        k.as_strided((B, k.shape[2], D), (k.stride(0), D, 1))
-    v3 = v.reshape(B, v.shape[2], D) if not (v.stride(3) == 1 and v.stride(2) == D) else \
-        v.as_strided((B, v.shape[2], D), (v.stride(0), D, 1))
-    _require(tuple(k3.shape[1:]) == (hkv, D), "k/v head shape must match the cache")
-    ks, vs = _token_rows(k3, "k"), _token_rows(v3, "v")
+    kshape = k.shape
+    if kshape != v.shape or kshape[0] != B or kshape[1] != 1:
+        raise RuntimeError("k/v must be [B, 1, Hkv, D]")
+    if k.dtype is not q.dtype or v.dtype is not q.dtype:
+        raise RuntimeError("k/v dtype mismatch")
+    if len(kshape) != 4 or kshape[2] != hkv or kshape[3] != D:
+        raise RuntimeError("k/v head shape must match the cache")
+    kst, vst = k.stride(), v.stride()
+    if kst[3] != 1 or kst[2] != D:  # heads and dims of a token side by side
+        k = k.reshape(B, hkv, D).contiguous()
+        kst = (hkv * D,)
+    if vst[3] != 1 or vst[2] != D:
+        v = v.reshape(B, hkv, D).contiguous()
+        vst = (hkv * D,)
+    ks, vs = (kst[0], vst[0]) if B > 1 else (hkv * D, hkv * D)
     rc = L.aac_decode_append_paged(
-        q3.data_ptr(), q3.stride(0), k3.data_ptr(), v3.data_ptr(), ks, vs, k_cache.data_ptr(),
+        q3.data_ptr(), q_stride, k.data_ptr(), v.data_ptr(), ks, vs, k_cache.data_ptr(),
         v_cache.data_ptr(), nblk, bs, tables.data_ptr(), mb, seqlens.data_ptr(), B, mcl, Hq, hkv,
         D, _scale(softmax_scale, D), out.data_ptr(), Hq * D, wsp, ws_bytes, part,
         _dtype_code(q), _stream(q))

@@ -8,13 +8,10 @@ from typing import Optional
 import torch
 
 from . import _lib
+from .flash_attn_interface import _stream
 
 __all__ = ["rmsnorm", "qk_norm_rope_store", "qkv_norm_rope_store", "silu_mul", "linear",
            "linear_supported", "rmsnorm_supported", "rmsnorm_linear", "argmax"]
-
-
-def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def _req(cond: bool, msg: str):
