@@ -257,10 +257,59 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
   // a few long ones running alone at the end.
   const int b = a.lpt ? __builtin_amdgcn_readfirstlane(seq_of_rank(a, blockIdx.z, tid))
                      : (int)blockIdx.z;  // wave-uniform (SGPR) either way
+  constexpr int R = 16;  // token rows of the workgroup (one per DPP row)
+  const int lane = tid & 63, wave = tid >> 6;
+  const int li = lane & 15, grp = lane >> 4;
+  const int rslot = wave * 4 + grp;  // 0 .. R - 1
+  const int t0 = part * a.part_tokens;
+  const int32_t* bt = a.block_tables + (int64_t)b * a.max_blocks;
+  const uint32_t nb32 = a.num_blocks < 0x7fffffff ? (uint32_t)a.num_blocks : 0x7fffffffu;
+  auto block_index = [&](int t) {
+    return POW2 ? t >> a.bs_shift : (int)(((uint64_t)(uint32_t)t * a.bs_magic) >> a.bs_mshift);
+  };
+
+  // A call of few sequences is a chain of latencies, so everything that does not
+  // depend on the context length is loaded beside it: the block numbers of the
+  // first iteration (clamped to the table; past the context replaced below)
+  // and the query rows.  The first K/V loads then wait for one load, not four,
+  // and the query's preparation runs while they are in flight (28-layer step of
+  // 4 sequences 879 -> 870 us; 256 x 1-2k 241.2 -> 240.2, 64 x 16k-32k 989.5 -> 984.5).
+  int blk[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) blk[u] = bt[min(block_index(t0 + rslot + R * u), a.max_blocks - 1)];
+  const int blk0 = bt[min(block_index(t0), a.max_blocks - 1)];
+  Raw8<DT> qr[G];
+  {
+    const char* qb = reinterpret_cast<const char*>(a.q) +
+                     ((int64_t)b * a.q_seq_stride + (int64_t)h * G * kHeadDim + li * 8) * ES;
+#pragma unroll
+    for (int g = 0; g < G; ++g) qr[g].load(qb + (int64_t)g * kHeadDim * ES);
+  }
+  // NEW == kQkv: the norm weight and RoPE rows of the query heads
+  u32x4 wraw, craw, sraw;
+  int64_t rope = 0;
+  if constexpr (NEW == kQkv) {
+    const int pos = a.positions[b];
+    rope = (int64_t)(pos < 0 ? 0 : (pos >= a.max_pos ? a.max_pos - 1 : pos)) * kHeadDim + li * 8;
+    wraw = *reinterpret_cast<const u32x4*>(a.qw + li * 8);
+    craw = *reinterpret_cast<const u32x4*>(a.cos + rope);
+    sraw = *reinterpret_cast<const u32x4*>(a.sin + rope);
+  }
+  // RMSNorm + RoPE of one head row
+  auto new_head = [&](const u32x4& raw, const u32x4& w) {
+    u32x4 o = raw;
+    if constexpr (NEW == kQkv) {
+      float wf[8], cf[8], sf[8];
+      fz::unpack8<DT>(w, wf);
+      fz::unpack8<DT>(craw, cf);
+      fz::signed_sin<DT>(sraw, li, sf);
+      o = fz::norm_rope_row<DT>(raw, a.eps, wf, cf, sf);
+    }
+    return o;
+  };
+
   const int ctx = context_len(a, b);
   const int np = parts_of(a, ctx);
-  constexpr int R = 16;  // token rows of the workgroup (one per DPP row)
-
   if (part >= np) {
     if (part == 0) {  // empty context: zeros (FA2 convention)
       for (int i = tid; i < G * (kHeadDim / 2); i += 256) {
@@ -271,31 +320,29 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
     }
     return;
   }
-  const int t0 = part * a.part_tokens;
-  int t1 = (part == np - 1) ? ctx : t0 + a.part_tokens;
+  // NEW: the last partition takes the new token (position lens[b], unless that
+  // lies outside the table) apart from the loop, which ends before it.
+  const bool has_new = NEW != kNone && part == np - 1 && a.lens[b] == ctx - 1;
+  const int t1 = (part == np - 1) ? ctx - (has_new ? 1 : 0) : t0 + a.part_tokens;
 
-  const int lane = tid & 63, wave = tid >> 6;
-  const int li = lane & 15, grp = lane >> 4;
-  const int rslot = wave * 4 + grp;  // 0 .. R - 1
+  const int64_t tok_bytes = (int64_t)a.hkv * kHeadDim * ES;  // cache row stride
+  const char* kbase = reinterpret_cast<const char*>(a.k_cache) + ((int64_t)h * kHeadDim + li * 8) * ES;
+  const char* vbase = reinterpret_cast<const char*>(a.v_cache) + ((int64_t)h * kHeadDim + li * 8) * ES;
 
-  // NEW == kQkv: norm + rotation of one head row.  `dim` is opaque, so that the
-  // new key's use of the norm and RoPE rows at the end of the loop reads them
-  // again instead of holding them in registers through it.
-  auto new_head = [&](const u32x4& raw, const u16* w) {
-    u32x4 o = raw;
-    if constexpr (NEW == kQkv) {
-      int dim = li * 8;
-      asm volatile("" : "+v"(dim));
-      const int pos = a.positions[b];
-      const int64_t p = (int64_t)(pos < 0 ? 0 : (pos >= a.max_pos ? a.max_pos - 1 : pos)) * kHeadDim + dim;
-      float wf[8], cf[8], sf[8];
-      fz::unpack8<DT>(*reinterpret_cast<const u32x4*>(w + dim), wf);
-      fz::unpack8<DT>(*reinterpret_cast<const u32x4*>(a.cos + p), cf);
-      fz::signed_sin<DT>(a.sin + p, li, sf);
-      o = fz::norm_rope_row<DT>(raw, a.eps, wf, cf, sf);
-    }
-    return o;
+  // Token t of this partition, or t0 (a valid token whose row is finite and
+  // whose probability is set to 0) past its end, so loads never branch.
+  auto token = [&](int t) { return t < t1 ? t : t0; };
+  // byte offset of token t's cache row in block `b` (bad entries read block 0)
+  auto row_off = [&](int t, int b) {
+    const int off = POW2 ? t & (a.block_size - 1) : t - block_index(t) * a.block_size;
+    return ((int64_t)((uint32_t)b < nb32 ? (uint32_t)b : 0u) * a.block_size + off) * tok_bytes;
   };
+  // The block numbers of an iteration's U tokens are loaded one iteration
+  // ahead: a block-table load waited for right before the K/V loads would,
+  // with in-order load counters, also wait for every K/V load issued before
+  // it and leave one token per wave in flight.
+#pragma unroll
+  for (int u = 0; u < U; ++u) blk[u] = t0 + rslot + R * u < t1 ? blk[u] : blk0;
 
   // q for the G heads of this KV head.  fp32: unpacked and pre-scaled into
   // the log2 domain.  bf16/fp16 (PK): kept packed and exact for v_dot2; the
@@ -303,100 +350,79 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
   constexpr bool PK = DT != Dt::FP32;
   float qf[PK ? 1 : G][8];
   u32 qp[PK ? G : 1][4];
-  {
-    const char* qb = reinterpret_cast<const char*>(a.q) +
-                     ((int64_t)b * a.q_seq_stride + (int64_t)h * G * kHeadDim + li * 8) * ES;
+  float m[G], l[G], acc[G][8];
+  // the query: once a row's first K/V loads are on their way, or before them
+  // where its registers beside theirs would spill
+  constexpr bool kQueryFirst = NEW == kQkv || G == 8 || DT == Dt::FP32;
+  auto prepare = [&]() {
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-      Raw8<DT> r;
-      r.load(qb + (int64_t)g * kHeadDim * ES);
-      if constexpr (NEW == kQkv) {
-        r.w[0] = new_head(r.w[0], a.qw);
-      }
+      if constexpr (NEW == kQkv) qr[g].w[0] = new_head(qr[g].w[0], wraw);
       if constexpr (PK) {
 #pragma unroll
-        for (int w = 0; w < 4; ++w) qp[g][w] = r.w[0][w];
+        for (int w = 0; w < 4; ++w) qp[g][w] = qr[g].w[0][w];
       } else {
-        r.unpack(qf[g]);
+        qr[g].unpack(qf[g]);
 #pragma unroll
         for (int i = 0; i < 8; ++i) qf[g][i] *= a.scale_log2;
       }
     }
-  }
 
-  float m[G], l[G], acc[G][8];
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-    m[g] = -1e30f;
-    l[g] = 0.f;
+    for (int g = 0; g < G; ++g) {
+      m[g] = -1e30f;
+      l[g] = 0.f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) acc[g][i] = 0.f;
-  }
-
-  const int64_t tok_bytes = (int64_t)a.hkv * kHeadDim * ES;  // cache row stride
-  const char* kbase = reinterpret_cast<const char*>(a.k_cache) + ((int64_t)h * kHeadDim + li * 8) * ES;
-  const char* vbase = reinterpret_cast<const char*>(a.v_cache) + ((int64_t)h * kHeadDim + li * 8) * ES;
-  const int32_t* bt = a.block_tables + (int64_t)b * a.max_blocks;
-  const uint32_t nb32 = a.num_blocks < 0x7fffffff ? (uint32_t)a.num_blocks : 0x7fffffffu;
-
-  // Token t of this partition, or t0 (a valid token whose row is finite and
-  // whose probability is set to 0) past its end, so loads never branch.
-  auto token = [&](int t) { return t < t1 ? t : t0; };
-  auto block_index = [&](int t) {
-    return POW2 ? t >> a.bs_shift : (int)(((uint64_t)(uint32_t)t * a.bs_magic) >> a.bs_mshift);
+      for (int i = 0; i < 8; ++i) acc[g][i] = 0.f;
+    }
   };
-  // The block numbers of an iteration's U tokens are loaded one iteration
-  // ahead: a block-table load waited for right before the K/V loads would,
-  // with in-order load counters, also wait for every K/V load issued before
-  // it and leave one token per wave in flight.
-  int blk[U];
 
-  // NEW: the last partition's first row starts from the new token, whose K and V
-  // it also writes to the caches; the loop ends before it.  Not appended past
-  // the table or to a block outside the cache (the loop then reads what the
-  // caches hold, as for kNone).
-  if constexpr (NEW != kNone) {
-    const int pos = a.lens[b];
-    if (part == np - 1 && pos == ctx - 1) {
-      const int bi = block_index(pos), bk = bt[bi];
-      if ((uint32_t)bk < nb32) {
-        t1 = pos;
-        if (wave == 0) {
-          Raw8<DT> kx, vx;
-          kx.load(reinterpret_cast<const char*>(a.k_new) + ((int64_t)b * a.k_new_stride + (int64_t)h * kHeadDim + li * 8) * ES);
-          vx.load(reinterpret_cast<const char*>(a.v_new) + ((int64_t)b * a.v_new_stride + (int64_t)h * kHeadDim + li * 8) * ES);
-          if constexpr (NEW == kQkv) kx.w[0] = new_head(kx.w[0], a.kw);
-          float vf[8], kf[PK ? 1 : 8];
-          vx.unpack(vf);
-          if constexpr (!PK) kx.unpack(kf);
-          const bool first = lane < kRowLanes;
+  bool ready = kQueryFirst;
+  if constexpr (kQueryFirst) prepare();
+
+  // The new token: row 0 of the workgroup starts its online softmax from the
+  // given rows and writes them to the caches (not to a block outside the
+  // cache: then the row that a bad entry reads takes their place).
+  if (NEW != kNone && has_new && wave == 0) {
+    if constexpr (!kQueryFirst) {
+      prepare();
+      ready = true;
+    }
+    const int pos = ctx - 1, bk = bt[block_index(pos)];
+    const bool store = (uint32_t)bk < nb32;  // wave-uniform
+    const int64_t off = row_off(pos, bk);
+    const int64_t hd = (int64_t)h * kHeadDim + li * 8;
+    Raw8<DT> kx, vx;
+    kx.load(store ? reinterpret_cast<const char*>(a.k_new) + (b * a.k_new_stride + hd) * ES : kbase + off);
+    vx.load(store ? reinterpret_cast<const char*>(a.v_new) + (b * a.v_new_stride + hd) * ES : vbase + off);
+    if constexpr (NEW == kQkv) {
+      if (store) kx.w[0] = new_head(kx.w[0], *reinterpret_cast<const u32x4*>(a.kw + li * 8));
+    }
+    float vf[8], kf[PK ? 1 : 8];
+    vx.unpack(vf);
+    if constexpr (!PK) kx.unpack(kf);
+    const bool first = lane < kRowLanes;
 #pragma unroll
-          for (int g = 0; g < G; ++g) {
-            float d = 0.f;
-            if constexpr (PK) {
+    for (int g = 0; g < G; ++g) {
+      float d = 0.f;
+      if constexpr (PK) {
 #pragma unroll
-              for (int w = 0; w < 4; ++w) d = Elem<DT>::dot2(kx.w[0][w], qp[g][w], d);
-            } else {
+        for (int w = 0; w < 4; ++w) d = Elem<DT>::dot2(kx.w[0][w], qp[g][w], d);
+      } else {
 #pragma unroll
-              for (int i = 0; i < 8; ++i) d = fmaf(qf[g][i], kf[i], d);
-            }
-            d = row16_sum(d);
-            m[g] = first ? (PK ? d * a.scale_log2 : d) : m[g];
-            l[g] = first ? 1.f : 0.f;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) acc[g][i] = first ? vf[i] : 0.f;
-          }
-          if (first) {
-            const int64_t off = ((int64_t)bk * a.block_size + (pos - bi * a.block_size)) * tok_bytes;
-            kx.store(const_cast<char*>(kbase) + off);
-            vx.store(const_cast<char*>(vbase) + off);
-          }
-        }
+        for (int i = 0; i < 8; ++i) d = fmaf(qf[g][i], kf[i], d);
       }
+      d = row16_sum(d);
+      m[g] = first ? (PK ? d * a.scale_log2 : d) : m[g];
+      l[g] = first ? 1.f : 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc[g][i] = first ? vf[i] : 0.f;
+    }
+    if (first && store) {
+      kx.store(const_cast<char*>(kbase) + off);
+      vx.store(const_cast<char*>(vbase) + off);
     }
   }
-#pragma unroll
-  for (int u = 0; u < U; ++u) blk[u] = bt[block_index(token(t0 + rslot + R * u))];
 
   for (int tb = t0 + rslot; tb < t1; tb += R * U) {
     Raw8<DT> kr[U], vr[U];
@@ -404,19 +430,19 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       valid[u] = tb + R * u < t1;
-      const int t = token(tb + R * u);
-      const int bi = block_index(t);
-      const int off = POW2 ? t & (a.block_size - 1) : t - bi * a.block_size;
-      const uint32_t bk = (uint32_t)blk[u] < nb32 ? (uint32_t)blk[u] : 0u;  // bad entries read block 0
-      const int64_t row = (int64_t)bk * a.block_size + off;
-      kr[u].load(kbase + row * tok_bytes);
-      vr[u].load(vbase + row * tok_bytes);
+      const int64_t off = row_off(token(tb + R * u), blk[u]);
+      kr[u].load(kbase + off);
+      vr[u].load(vbase + off);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) blk[u] = bt[block_index(token(tb + R * U + R * u))];
     // Every load above is issued before any arithmetic below (the scheduler
     // would otherwise pull each token's math up behind its load and wait).
     __builtin_amdgcn_sched_barrier(0);
+    if (!kQueryFirst && !ready) {
+      prepare();
+      ready = true;
+    }
     float s[U][G];
     if constexpr (PK) {
       // Packed bf16/fp16: q.k with v_dot2 on the packed rows (no unpacking),
@@ -509,6 +535,7 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
       }
     }
   }
+  if (!kQueryFirst && !ready) prepare();
 
   // Merge the 4 DPP rows of this wave (lanes li, li+16, li+32, li+48 hold the
   // same dims).

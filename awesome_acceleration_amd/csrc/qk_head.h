@@ -186,10 +186,14 @@ __device__ __forceinline__ void norm_rope_head(const QkArgs& a, int64_t t, int h
 // sin of the lane's dims, negated in the first half: rounding is symmetric,
 // so (-partner) * sin and partner * (-sin) are the same bits.
 template <Dt DT>
-__device__ __forceinline__ void signed_sin(const u16* sin8, int li, float* sf) {
-  unpack8<DT>(*reinterpret_cast<const u32x4*>(sin8), sf);
+__device__ __forceinline__ void signed_sin(const u32x4& sin8, int li, float* sf) {
+  unpack8<DT>(sin8, sf);
 #pragma unroll
   for (int i = 0; i < 8; ++i) sf[i] = li < 8 ? -sf[i] : sf[i];
+}
+template <Dt DT>
+__device__ __forceinline__ void signed_sin(const u16* sin8, int li, float* sf) {
+  signed_sin<DT>(*reinterpret_cast<const u32x4*>(sin8), li, sf);
 }
 
 __device__ __forceinline__ int clamp_pos(const QkArgs& a, int p) {
