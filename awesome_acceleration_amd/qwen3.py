@@ -39,7 +39,16 @@ from . import paged
 __all__ = ["Qwen3Config", "Qwen3ForCausalLM", "PagedKVCache", "StepMeta"]
 
 
-NORM_GEMM_ROWS = 16
+# Where the forms of a decode step change hands, in sequences (us a step of 14
+# Qwen3-0.6B layers on MI355X).  The norm inside the next projection's launch: 20
+# sequences 794 against 815, 32: 828 against 819.  q/k norm + RoPE in the attention
+# launch after a plain QKV projection, against the projection's epilogue: 20
+# sequences 815 against 853, 32: 819 against 875; 48: 996 against 986, and 256 (4
+# layers) 1040 against 1006, where the epilogue's 32-row tiles fill the GPU.
+NORM_GEMM_ROWS = 24
+QKV_ATTENTION_ROWS = 32
+# The lm_head (151,936 x 1024) on the few-row projection kernel, us against the
+# library: 1-4 rows 45.5 / 53, 8: 48.8 / 53, 16: 63.9 / 55.
 LM_HEAD_ROWS = 8
 
 
@@ -259,9 +268,10 @@ class Qwen3ForCausalLM:
         RMSNorm, q/k RMSNorm + RoPE + KV store/append, SiLU * up are one launch
         each, and the residual add of each block is folded into the next norm.
         A decode step's projections (one row per sequence) run on the
-        decode-batch GEMM, QKV with the q/k norm + RoPE + KV append and
-        gate/up with SiLU * up in their epilogues; prefill steps (many rows)
-        keep the library GEMMs."""
+        decode-batch GEMM, gate/up with SiLU * up in its epilogue; the q/k norm,
+        RoPE and KV append run in the attention launch or, from
+        QKV_ATTENTION_ROWS on, in QKV's epilogue; prefill steps (many rows) keep
+        the library GEMMs."""
         eps = self.cfg.rms_norm_eps
         I = self.cfg.intermediate_size
         h = F.embedding(input_ids, self.embed)
@@ -271,47 +281,40 @@ class Qwen3ForCausalLM:
         small = not prefill and T <= self.small_gemm_rows
         lin = fz.linear if small else F.linear
         merged = small and T <= self.norm_gemm_rows
+        epilogue = small and T > QKV_ATTENTION_ROWS
         for li, L in enumerate(self.layers):
-            if merged:
-                # norm + projection, then q/k norm + RoPE, KV append and attention
+            if merged:  # norm and projection in one launch
                 qkv, r = fz.rmsnorm_linear(res if delta is None else delta, L["ln1"], eps, L["qkv"],
                                            residual=None if delta is None else res)
                 res = res if delta is None else r
-                attn = fai.decode_qkv_paged(
-                    qkv, self.hq, L["q_norm"], L["k_norm"], eps, self.rope.cos, self.rope.sin, pos,
-                    cache.k(li), cache.v(li), meta.block_tables, meta.cache_seqlens,
-                    softmax_scale=self.scale, max_context_len=meta.max_context_len)
-            elif delta is None:
-                x = fz.rmsnorm(res, L["ln1"], eps)
             else:
-                x, res = fz.rmsnorm(delta, L["ln1"], eps, residual=res)
-            if merged:
-                pass
-            elif small:  # projection, q/k norm + RoPE and the KV append in one launch
+                if delta is None:
+                    x = fz.rmsnorm(res, L["ln1"], eps)
+                else:
+                    x, res = fz.rmsnorm(delta, L["ln1"], eps, residual=res)
+                if not epilogue:
+                    qkv = lin(x, L["qkv"])
+            if prefill:
+                q, k = fz.qk_norm_rope_store(
+                    qkv, self.hq, self.hkv, L["q_norm"], L["k_norm"], eps, self.rope.cos,
+                    self.rope.sin, pos, cache.k(li), cache.v(li), slot_mapping=meta.slot_mapping)
+                v = qkv[:, self.q_size + self.kv_size:].view(T, self.hkv, self.d)
+                attn = fai.flash_attn_varlen_func(q, k, v, meta.cu_seqlens, meta.cu_seqlens,
+                                                  meta.max_seqlen, meta.max_seqlen,
+                                                  softmax_scale=self.scale, causal=True)
+            elif epilogue:  # projection, q/k norm + RoPE and the KV append in one launch
                 q, _ = fz.qkv_norm_rope_store(
                     x, L["qkv"], self.hq, self.hkv, L["q_norm"], L["k_norm"], eps, self.rope.cos,
                     self.rope.sin, pos, cache.k(li), cache.v(li), block_tables=meta.block_tables,
                     cache_seqlens=meta.cache_seqlens, want_k=False)
-            else:
-                qkv = F.linear(x, L["qkv"])
-                if prefill:
-                    q, k = fz.qk_norm_rope_store(
-                        qkv, self.hq, self.hkv, L["q_norm"], L["k_norm"], eps, self.rope.cos,
-                        self.rope.sin, pos, cache.k(li), cache.v(li), slot_mapping=meta.slot_mapping)
-                    v = qkv[:, self.q_size + self.kv_size:].view(T, self.hkv, self.d)
-                    attn = fai.flash_attn_varlen_func(q, k, v, meta.cu_seqlens, meta.cu_seqlens,
-                                                      meta.max_seqlen, meta.max_seqlen,
-                                                      softmax_scale=self.scale, causal=True)
-                else:
-                    q, _ = fz.qk_norm_rope_store(
-                        qkv, self.hq, self.hkv, L["q_norm"], L["k_norm"], eps, self.rope.cos,
-                        self.rope.sin, pos, cache.k(li), cache.v(li),
-                        block_tables=meta.block_tables, cache_seqlens=meta.cache_seqlens,
-                        want_k=False)
-            if not prefill and not merged:
                 attn = fai.decode_paged(q, cache.k(li), cache.v(li), meta.block_tables,
                                         meta.context_lens, softmax_scale=self.scale,
                                         max_context_len=meta.max_context_len)
+            else:  # q/k norm + RoPE, the KV append and the attention in one launch
+                attn = fai.decode_qkv_paged(
+                    qkv, self.hq, L["q_norm"], L["k_norm"], eps, self.rope.cos, self.rope.sin, pos,
+                    cache.k(li), cache.v(li), meta.block_tables, meta.cache_seqlens,
+                    softmax_scale=self.scale, max_context_len=meta.max_context_len)
             o = lin(attn.reshape(T, -1), L["o"])
             if merged:
                 act, res = fz.rmsnorm_linear(o, L["ln2"], eps, L["gate_up"], residual=res, silu=True)
@@ -325,9 +328,7 @@ class Qwen3ForCausalLM:
         if prefill:
             delta, res = delta[meta.last_idx], res[meta.last_idx]
         h, _ = fz.rmsnorm(delta, self.norm, eps, residual=res)
-        # tied embeddings; up to LM_HEAD_ROWS rows the streaming kernel of the
-        # few-row projections (hidden 1024, vocabulary 151,936, us against the
-        # library: 1-4 rows 46.0 / 53, 8 48.6 / 54, 16 64.2 / 55)
+        # tied embeddings
         if merged and T <= LM_HEAD_ROWS and self.embed.shape[0] % 32 == 0:
             return fz.linear(h, self.embed)
         return F.linear(h, self.embed)
