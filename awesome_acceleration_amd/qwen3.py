@@ -302,11 +302,17 @@ class Qwen3ForCausalLM:
                 attn = fai.flash_attn_varlen_func(q, k, v, meta.cu_seqlens, meta.cu_seqlens,
                                                   meta.max_seqlen, meta.max_seqlen,
                                                   softmax_scale=self.scale, causal=True)
-            elif epilogue:  # projection, q/k norm + RoPE and the KV append in one launch
-                q, _ = fz.qkv_norm_rope_store(
-                    x, L["qkv"], self.hq, self.hkv, L["q_norm"], L["k_norm"], eps, self.rope.cos,
-                    self.rope.sin, pos, cache.k(li), cache.v(li), block_tables=meta.block_tables,
-                    cache_seqlens=meta.cache_seqlens, want_k=False)
+            elif T > QKV_ATTENTION_ROWS:
+                # q/k norm + RoPE and the KV append, in the projection's launch
+                # where the decode-batch GEMM takes it
+                norms = (self.hq, self.hkv, L["q_norm"], L["k_norm"], eps, self.rope.cos,
+                         self.rope.sin, pos, cache.k(li), cache.v(li))
+                append = dict(block_tables=meta.block_tables, cache_seqlens=meta.cache_seqlens,
+                              want_k=False)
+                if epilogue:
+                    q, _ = fz.qkv_norm_rope_store(x, L["qkv"], *norms, **append)
+                else:
+                    q, _ = fz.qk_norm_rope_store(qkv, *norms, **append)
                 attn = fai.decode_paged(q, cache.k(li), cache.v(li), meta.block_tables,
                                         meta.context_lens, softmax_scale=self.scale,
                                         max_context_len=meta.max_context_len)
