@@ -779,13 +779,13 @@ static int prefill_common(const void* q, const void* k, const void* v, int64_t q
   pf::SplitPlan sp = {1, 0, 0};
   if (n_store == 0 && workspace && (uintptr_t)workspace % 256 == 0)
     sp = pf::plan_split(n_seqs, max_seqlen_q, max_seqlen_k, n_q_heads, n_kv_heads, causal != 0, n_cu);
-  // the split kernel's loads may reach 128 rows past a segment's keys: their
-  // (out of range) offsets stay in 32 bits
-  const bool few = prefill_split_takes(g, scale, n_seqs, n_kv_heads, max_seqlen_q, max_seqlen_k, n_cu) &&
-                   ((int64_t)max_seqlen_k + 160) * std::max(k_tok_stride, v_tok_stride) * 2 <
-                       (int64_t(1) << 31);
-  if (few) {
-    rc = prefill_split_launch(a, g, causal != 0, n_store > 0, f16, max_seqlen_q, stream);
+  // that kernel's loads may reach 128 rows past a segment's keys: their (out of
+  // range) offsets stay in 32 bits
+  const bool reach = ((int64_t)max_seqlen_k + 160) * std::max(k_tok_stride, v_tok_stride) * 2 < (int64_t(1) << 31);
+  const int slices =
+      reach ? prefill_split_slices(g, scale, n_seqs, n_kv_heads, max_seqlen_q, max_seqlen_k, n_cu) : 0;
+  if (slices) {
+    rc = prefill_split_launch(a, slices, g, causal != 0, n_store > 0, f16, max_seqlen_q, stream);
   } else if (sp.n_split > 1 && workspace_bytes >= sp.ws_bytes) {
     a.n_split = sp.n_split;
     a.ws_cnt = reinterpret_cast<int32_t*>(workspace);

@@ -8,18 +8,21 @@
 // queries at G = 2, every key of its KV head in turn) makes 56 items of up to
 // 13 tiles from 777 tokens at 16/8 heads, on 256 CUs.  Here an item is 32
 // queries of two query heads of a KV head, and the keys are split over the
-// workgroup's waves: wave (c, s) takes head c and the 32-key sub-tiles s, s + 4,
-// s + 8, ..., so the chain is a sixteenth of the context's sub-tiles per
-// 128 keys.  Two waves per SIMD run the two heads of a slice, one's softmax
-// beside the other's MFMAs.  The four partial results of a head (reference
-// max, row sum, O) are merged through LDS at the end.
+// workgroup's waves: with SL slices, wave (c, s) takes head c and the 32-key
+// sub-tiles s, s + SL, s + 2 SL, ...  The partial results of a head (reference
+// max, row sum, O) are merged through LDS at the end.  Two forms:
+//   SL = 4: eight waves, two LDS stages of 128 keys, one workgroup per CU: the
+//     shortest chain, for fewer items than CUs.  Two waves per SIMD run the two
+//     heads of a slice, one's softmax beside the other's MFMAs.
+//   SL = 2: four waves, one stage of 64 keys, three workgroups per CU: one's
+//     loads, merge and stores run beside the others' products.  For short
+//     segments and a few items per CU.
 //
-// Tiles: per iteration the workgroup stages 128 keys of K and V (64 KiB)
-// straight from global memory into one of two LDS stages; wave (0, s) brings
-// slice s's K rows, wave (1, s) its V rows.  One barrier per iteration: past it
-// every wave's tile has landed and the other stage is free for the next loads.
-// Row layouts, fragments, masks, lazy rescaling and the probability rounding
-// are those of prefill_wide.hip.
+// Tiles go straight from global memory into LDS; wave (0, s) brings slice s's
+// K rows, wave (1, s) its V rows.  With two stages there is one barrier per
+// iteration: past it every wave's tile has landed and the other stage is free
+// for the next loads.  Row layouts, fragments, masks, lazy rescaling and the
+// probability rounding are those of prefill_wide.hip.
 
 #include <algorithm>
 
@@ -33,14 +36,21 @@ using pf::Args;
 using pf::D;
 using pf::kRescale;
 
-constexpr int kWaves = 8, kThreads = 64 * kWaves;
-constexpr int kSlices = 4;                  // key slices (32 keys each per iteration)
-constexpr int kSubBytes = 32 * D * 2;       // 8 KiB: a sub-tile of K or V
-constexpr int kStageBytes = kSlices * 2 * kSubBytes;
-constexpr int kOutPitch = D * 2 + 16;       // bytes of an output staging row
-constexpr int kOutOff = 2 * kStageBytes;    // [2 heads][32 queries]
-constexpr int kMlOff = kOutOff + 2 * 32 * kOutPitch;
-constexpr int kLdsBytes = kMlOff + kWaves * 32 * 8;
+constexpr int kSubBytes = 32 * D * 2;   // 8 KiB: a sub-tile of K or V
+constexpr int kOutPitch = D * 2 + 16;   // bytes of an output staging row
+
+// SL key slices (32 keys each per iteration) on 2 SL waves, STAGES LDS stages.
+template <int SL, int STAGES> struct Shape {
+  static constexpr int kWaves = 2 * SL, kThreads = 64 * kWaves;
+  static constexpr int kStageBytes = SL * 2 * kSubBytes;
+  // partial O of the merge, over the dead stages: 4 KiB per 32 dims that a wave
+  // hands to another slice's
+  static constexpr int kPartBytes = kWaves * (SL == 4 ? 4 : 2) * 4096;
+  static constexpr int kTiles = STAGES * kStageBytes > kPartBytes ? STAGES * kStageBytes : kPartBytes;
+  static constexpr int kOutOff = kTiles;  // [2 heads][32 queries]
+  static constexpr int kMlOff = kOutOff + 2 * 32 * kOutPitch;
+  static constexpr int kLdsBytes = kMlOff + kWaves * 32 * 8;
+};
 
 typedef __attribute__((address_space(3))) unsigned char lds_u8;
 typedef short v4s __attribute__((ext_vector_type(4)));
@@ -64,11 +74,15 @@ __device__ __forceinline__ void landed_barrier() {
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-template <bool CAUSAL, bool STORE, bool F16>
-__global__ __launch_bounds__(kThreads, 1) void prefill_split_kernel(Args a) {
+template <int SL, int STAGES, bool CAUSAL, bool STORE, bool F16>
+__global__ __launch_bounds__(128 * SL, SL == 4 ? 2 : 3) void prefill_split_kernel(Args a) {
   static_assert(CAUSAL || !STORE, "the store variant is causal self-attention");
+  static_assert((SL == 4 && STAGES == 2) || (SL == 2 && STAGES == 1), "the two forms");
   typedef pf::Mfma<F16> M;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[kLdsBytes];
+  typedef Shape<SL, STAGES> S;
+  constexpr int kThreads = S::kThreads, kSlices = SL, kStageBytes = S::kStageBytes;
+  constexpr int kOutOff = S::kOutOff, kMlOff = S::kMlOff;
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[S::kLdsBytes];
   const u32 lds0 = (u32)(uintptr_t)(lds_u8*)lds;
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -121,7 +135,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_split_kernel(Args a) {
     const int key0 = 32 * (n * kSlices + sl);
 #pragma unroll
     for (int i = 0; i < 8; ++i)
-      load_lds16(rs, voff[i & 3], (key0 + 4 * i) * row_bytes, dst0 + (u32)((n & 1) * kStageBytes + i * 1024));
+      load_lds16(rs, voff[i & 3], (key0 + 4 * i) * row_bytes, dst0 + (u32)(n % STAGES * kStageBytes + i * 1024));
   };
   if (n_it > 0) issue(0);
 
@@ -152,11 +166,19 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_split_kernel(Args a) {
   float m = -1e30f, l = 0.f;  // reference max (raw scores), lane-partial row sum
 
   for (int n = 0; n < n_it; ++n) {
-    landed_barrier();
-    if (n + 1 < n_it) issue(n + 1);
+    if constexpr (STAGES == 1) {
+      if (n > 0) {
+        __syncthreads();  // every wave is done with the tile before
+        issue(n);
+      }
+      landed_barrier();
+    } else {
+      landed_barrier();
+      if (n + 1 < n_it) issue(n + 1);
+    }
     const int j = n * kSlices + sl;
     if (j >= nsub) continue;  // the last iteration's slices past the end
-    const lds_u8* kb = (const lds_u8*)lds + (n & 1) * kStageBytes + sl * 2 * kSubBytes;
+    const lds_u8* kb = (const lds_u8*)lds + n % STAGES * kStageBytes + sl * 2 * kSubBytes;
     const lds_u8* vb = kb + kSubBytes;
     f32x16 s;
 #pragma unroll
@@ -207,76 +229,101 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_split_kernel(Args a) {
   }
 
   // KV-cache store: the item's own 32 rows taken as keys (one pair per KV
-  // head), loaded here and written after the output
-  u32x4 ok[2];
-  int64_t oslot = -1;
-  const int orow = tid >> 4, och = (tid & 15) * 8;  // 32 rows x 16 chunks
+  // head), loaded here and written after the output: 16 threads a row
+  constexpr int kRows = kThreads / 16, kPass = 32 / kRows;
+  u32x4 ok[kPass], ov[kPass];
+  int64_t oslot[kPass];
+  const int orow = tid >> 4, och = (tid & 15) * 8;
   if constexpr (STORE) {
-    const int64_t tok = (int64_t)k_beg + q0 + orow;
-    if (pr == 0 && q0 + orow < Lq && tok < a.n_tok) {
-      oslot = a.slots[tok];
-      ok[0] = *reinterpret_cast<const u32x4*>(a.k + tok * a.k_stride + h * D + och);
-      ok[1] = *reinterpret_cast<const u32x4*>(a.v + tok * a.v_stride + h * D + och);
+#pragma unroll
+    for (int i = 0; i < kPass; ++i) {
+      const int row = q0 + orow + i * kRows;
+      const int64_t tok = (int64_t)k_beg + row;
+      oslot[i] = -1;
+      if (pr == 0 && row < Lq && tok < a.n_tok) {
+        oslot[i] = a.slots[tok];
+        ok[i] = *reinterpret_cast<const u32x4*>(a.k + tok * a.k_stride + h * D + och);
+        ov[i] = *reinterpret_cast<const u32x4*>(a.v + tok * a.v_stride + h * D + och);
+      }
     }
   }
 
-  // merge the four slices of each head: partial O over the (dead) stages,
-  // [wave][16 float4][64 lanes]; then wave (c, s) sums dims 32 s .. + 31
+  // Merge the slices of each head: slice s takes dims 128 s / SL and up, its own
+  // part from registers, the others' through LDS (over the dead stages).
   {
     const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
     l = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
   }
+  auto part = [&](int w, int db) {  // 4 KiB of wave w's dims 32 db .. + 31: [4][64 lanes]
+    return reinterpret_cast<f32x4*>(lds + (SL == 4 ? 4 * w + db : 2 * w + (db & 1)) * 4096);
+  };
   __syncthreads();
   float2* ml = reinterpret_cast<float2*>(lds + kMlOff);
   if (lane < 32) ml[wave * 32 + col] = make_float2(m, l);
-  f32x4* part = reinterpret_cast<f32x4*>(lds + wave * 16384);
 #pragma unroll
   for (int db = 0; db < 4; ++db)
+    if (db * SL / 4 != sl) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      part[(4 * db + r) * 64 + lane] = f32x4{o[db][4 * r], o[db][4 * r + 1], o[db][4 * r + 2], o[db][4 * r + 3]};
+      for (int r = 0; r < 4; ++r)
+        part(wave, db)[r * 64 + lane] = f32x4{o[db][4 * r], o[db][4 * r + 1], o[db][4 * r + 2], o[db][4 * r + 3]};
+    }
   __syncthreads();
-  float2 mls[kSlices];
+  float2 mls[SL];
   float mx = -1e30f;
 #pragma unroll
-  for (int k = 0; k < kSlices; ++k) {
+  for (int k = 0; k < SL; ++k) {
     mls[k] = ml[(2 * k + c) * 32 + col];
     mx = vmax(mx, mls[k].x);
   }
-  float wt[kSlices], lt = 0.f;
+  float wt[SL], lt = 0.f;
 #pragma unroll
-  for (int k = 0; k < kSlices; ++k) {
+  for (int k = 0; k < SL; ++k) {
     wt[k] = fast_exp2((mls[k].x - mx) * cs);
     lt = fmaf(mls[k].y, wt[k], lt);
   }
   const float inv = lt > 0.f ? __builtin_amdgcn_rcpf(lt) : 0.f;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int db = 0; db < 4; ++db)
+    if (db * SL / 4 == sl) {
 #pragma unroll
-    for (int k = 0; k < kSlices; ++k) {
-      const f32x4 x = *reinterpret_cast<const f32x4*>(lds + (2 * k + c) * 16384 + ((4 * sl + r) * 64 + lane) * 16);
+      for (int r = 0; r < 4; ++r) {
+        float v[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = fmaf(x[e], wt[k], v[e]);
+        for (int k = 0; k < SL; ++k) {  // in slice order
+          if (k == db * SL / 4) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = fmaf(o[db][4 * r + e], wt[k], v[e]);
+          } else {
+            const f32x4 x = part(2 * k + c, db)[r * 64 + lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = fmaf(x[e], wt[k], v[e]);
+          }
+        }
+        u32x2 w;
+        w[0] = M::pack(v[0] * inv, v[1] * inv);
+        w[1] = M::pack(v[2] * inv, v[3] * inv);
+        *reinterpret_cast<u32x2*>(lds + kOutOff + (c * 32 + col) * kOutPitch + (32 * db + 8 * r + 4 * hl) * 2) = w;
+      }
     }
-    u32x2 w;
-    w[0] = M::pack(v[0] * inv, v[1] * inv);
-    w[1] = M::pack(v[2] * inv, v[3] * inv);
-    *reinterpret_cast<u32x2*>(lds + kOutOff + (c * 32 + col) * kOutPitch + (32 * sl + 8 * r + 4 * hl) * 2) = w;
-  }
   __syncthreads();
-  if (q0 + orow < Lq) {
 #pragma unroll
-    for (int k = 0; k < 2; ++k)
-      *reinterpret_cast<u32x4*>(a.out + (int64_t)(q_beg + q0 + orow) * a.o_stride + (head + k) * D + och) =
-          *reinterpret_cast<const u32x4*>(lds + kOutOff + (k * 32 + orow) * kOutPitch + och * 2);
+  for (int i = 0; i < kPass; ++i) {
+    const int row = orow + i * kRows;
+    if (q0 + row < Lq) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+        *reinterpret_cast<u32x4*>(a.out + (int64_t)(q_beg + q0 + row) * a.o_stride + (head + k) * D + och) =
+            *reinterpret_cast<const u32x4*>(lds + kOutOff + (k * 32 + row) * kOutPitch + och * 2);
+    }
   }
   if constexpr (STORE) {
-    if (oslot >= 0 && oslot < a.num_rows) {
-      const int64_t dst = (oslot * a.hkv + h) * D + och;
-      *reinterpret_cast<u32x4*>(a.kc + dst) = ok[0];
-      *reinterpret_cast<u32x4*>(a.vc + dst) = ok[1];
-    }
+#pragma unroll
+    for (int i = 0; i < kPass; ++i)
+      if (oslot[i] >= 0 && oslot[i] < a.num_rows) {
+        const int64_t dst = (oslot[i] * a.hkv + h) * D + och;
+        *reinterpret_cast<u32x4*>(a.kc + dst) = ok[i];
+        *reinterpret_cast<u32x4*>(a.vc + dst) = ov[i];
+      }
     // q-blocks of the segment that no item owns (max_seqlen below its length)
     if (z == 0 && pr == 0 && nqb > a.n_qblocks)
       pf::store_kv_span<kThreads>(a, tid, k_beg, k_beg + (int64_t)(nqb - a.n_qblocks) * 32, h, h + 1);
@@ -284,37 +331,56 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_split_kernel(Args a) {
 }
 
 template <bool CAUSAL, bool STORE, bool F16>
-static void launch_t(const Args& a, unsigned grid, hipStream_t st) {
-  hipLaunchKernelGGL((prefill_split_kernel<CAUSAL, STORE, F16>), dim3(grid), dim3(kThreads), 0, st, a);
+static void launch_t(const Args& a, bool four, unsigned grid, hipStream_t st) {
+  if (four)
+    hipLaunchKernelGGL((prefill_split_kernel<4, 2, CAUSAL, STORE, F16>), dim3(grid), dim3(Shape<4, 2>::kThreads), 0, st, a);
+  else
+    hipLaunchKernelGGL((prefill_split_kernel<2, 1, CAUSAL, STORE, F16>), dim3(grid), dim3(Shape<2, 1>::kThreads), 0, st, a);
 }
 
 }  // namespace ps
 
-// Up to one item per CU the call runs here; up to two per CU from 512 keys on.
-// Measured (us, the other kernel -> this one; causal, graph replay): 16/8 heads,
-// one request of 128 tokens 11.5 -> 6.8, 777 23.3 -> 12.3 (with the store 24.8 ->
-// 13.3), 1024 28.6 -> 15.0, 2048 (512 items) 48.9 -> 31.3; 8 x 128 (256 items)
-// 12.0 -> 7.4; two items per CU: 4 x 512 18.8 -> 17.0 but 8 x 256 13.6 -> 14.7 and
-// 32 x 64 10.1 -> 13.1; four per CU: 1 x 4096 93 -> 97, 2 x 2048 54 -> 61, 8 x 512
-// 20 -> 33 (the wide kernel's tiles serve four times the queries).  32/8 and 8/4
-// heads lie alike at equal item counts.
-bool prefill_split_takes(int g, float scale, int n_seqs, int hkv, int max_q, int max_k, int n_cu) {
-  if ((g != 2 && g != 4 && g != 8) || !(scale > 0.f)) return false;
+// Where the lines lie, by items (32 queries of two heads) per CU.  Measured on
+// MI355X (causal, graph replay, us): W the wide kernel, 4 and 2 the slices here.
+//   up to one item: 16/8 heads, 1 x 128 W 11.5, 4 6.4, 2 5.7; 1 x 256 12.9, 7.5,
+//     7.5; 1 x 777 23.3, 12.1, 15.1 (with the store 24.8, 12.9); 1 x 1024 28.6,
+//     14.5, 18.9: four slices for more than 256 keys
+//   up to two: 4 x 512 W 18.9, 4 16.6, 2 13.1; 1 x 2048 48.7, 29.2, 33.6; 8/4 heads
+//     3 x 1024 28.4, 17.9, 19.3: four from 640 keys on
+//   up to three: 6 x 512 W 19.0, 2 15.9; 1 x 3072 69.1, 57.0; 12 x 250 13.1, 11.8
+//   up to four: 1 x 4096 W 93.1, 2 84.7; 2 x 2048 50.7, 47.8, but 16 x 256 15.2,
+//     18.0: from 1024 keys on.  Beyond, the wide kernel, whose tiles serve four
+//     times the queries (8 x 1024 46.4, 55.9)
+//   segments of one block of 32 queries keep one of its four waves busy: 256 x 32
+//     at 16/8 heads W 50.3, 2 21.6, at 32/8 55.5, 33.4; of two blocks 57.0, 40.8,
+//     but at 32/8 67.7, 82.0
+static int pick_slices(int g, int n_seqs, int hkv, int max_q, int max_k, int n_cu) {
   const int64_t items = (int64_t)n_seqs * hkv * (g / 2) * cdiv(max_q, 32);
-  return items <= n_cu || (items <= 2 * (int64_t)n_cu && max_k >= 512);
+  if ((items <= n_cu && max_k > 256) || (items <= 2 * (int64_t)n_cu && max_k >= 640)) return 4;
+  if (items <= 3 * (int64_t)n_cu || (items <= 4 * (int64_t)n_cu && max_k >= 1024) || max_q <= 32 ||
+      (max_q <= 64 && g == 2))
+    return 2;
+  return 0;
 }
 
-int prefill_split_launch(const pf::Args& a0, int g, bool causal, bool store, bool f16, int max_q, hipStream_t st) {
+int prefill_split_slices(int g, float scale, int n_seqs, int hkv, int max_q, int max_k, int n_cu) {
+  if ((g != 2 && g != 4 && g != 8) || !(scale > 0.f)) return 0;
+  return pick_slices(g, n_seqs, hkv, max_q, max_k, n_cu);
+}
+
+int prefill_split_launch(const pf::Args& a0, int slices, int g, bool causal, bool store, bool f16, int max_q,
+                         hipStream_t st) {
   if (store && !causal) return AAC_ERR_UNSUPPORTED;
   pf::Args a = a0;
   a.n_qblocks = (int)cdiv(max_q, 32);
   const unsigned grid = (unsigned)((int64_t)a.n_seqs * a.hkv * (g / 2) * a.n_qblocks);
+  const bool four = slices == 4;
   if (store) {
-    if (f16) ps::launch_t<true, true, true>(a, grid, st); else ps::launch_t<true, true, false>(a, grid, st);
+    if (f16) ps::launch_t<true, true, true>(a, four, grid, st); else ps::launch_t<true, true, false>(a, four, grid, st);
   } else if (causal) {
-    if (f16) ps::launch_t<true, false, true>(a, grid, st); else ps::launch_t<true, false, false>(a, grid, st);
+    if (f16) ps::launch_t<true, false, true>(a, four, grid, st); else ps::launch_t<true, false, false>(a, four, grid, st);
   } else {
-    if (f16) ps::launch_t<false, false, true>(a, grid, st); else ps::launch_t<false, false, false>(a, grid, st);
+    if (f16) ps::launch_t<false, false, true>(a, four, grid, st); else ps::launch_t<false, false, false>(a, four, grid, st);
   }
   return AAC_OK;
 }

@@ -427,13 +427,14 @@ def test_prefill_tile_edges_plain_and_stored(gpu, hq, hkv, dtype):
 @pytest.mark.parametrize("hq,hkv", [(16, 8), (16, 4), (16, 2)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("causal", [True, False])
-def test_prefill_few_queries(gpu, hq, hkv, dtype, causal):
+@pytest.mark.parametrize("keys", [600, 200])  # the longest: four or two key slices
+def test_prefill_few_queries(gpu, hq, hkv, dtype, causal, keys):
     # few items: the keys split over a workgroup's waves.  Query counts around
     # the 32-row blocks, key counts around the 32-key sub-tiles and the 128-key
     # iterations, more and fewer keys than queries, empty segments, strided rows
     print(f"case: few queries {hq}/{hkv} {dtype} causal={causal}", flush=True)
     lq = [1, 31, 33, 64, 0, 5, 40, 32]
-    lk = [1, 31, 33, 129, 7, 600, 11, 0]
+    lk = [1, 31, 33, 129, 7, keys, 11, 0]
     q, k, v, cq, ck = _ragged(lq, lk, hq, hkv, dtype, gpu, 41)
     wide = torch.randn((sum(lk), 2 * hkv + 1, 128), device=gpu).to(dtype)
     wide[:, 1:hkv + 1], wide[:, hkv + 1:] = k, v
