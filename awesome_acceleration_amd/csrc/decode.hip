@@ -85,6 +85,8 @@ struct DecodeArgs {
   int64_t out_seq_stride;  // elements
   float* ws_o;             // [B][Hq][P][D] normalised partial outputs
   float* ws_lse;           // [B][Hq][P]    log2-sum-exp of each partition
+  // [B][Hkv] finished partitions, or null: a second launch combines them
+  unsigned long long* ws_cnt;
   int32_t n_parts;
   int32_t part_tokens;
   int32_t bs_shift;  // log2(block_size) when it is a power of two
@@ -112,7 +114,10 @@ struct DecodeArgs {
 // What the launch does with the step's new token: nothing (its rows are in the
 // caches already), append its K/V rows, or also make q and k from the QKV
 // projection's rows (q/k RMSNorm + RoPE).
-enum { kNone = 0, kAppend = 1, kQkv = 2 };
+// kAppendMerge: kAppend, and the partition that finishes last combines them all
+// (a form of its own, as its code costs the others 0.85 us a launch: a 28-layer
+// step of 4 sequences 872 -> 896 us).
+enum { kNone = 0, kAppend = 1, kQkv = 2, kAppendMerge = 3 };
 
 // Raw storage for the 8 elements one lane owns in one token row.
 template <Dt DT> struct Raw8 {
@@ -231,6 +236,18 @@ __device__ __forceinline__ void store_out2(void* out, int64_t idx, float x0, flo
   } else {
     *reinterpret_cast<u32*>(reinterpret_cast<u16*>(out) + idx) = Elem<DT>::pack2(x0, x1);
   }
+}
+
+// A (sequence, KV head)'s partial rows and log-sum-exps in the workspace
+constexpr int kSc1 = 16;  // cache policy: coherent across XCDs
+constexpr unsigned long long kCntTag = 0xa3c59e176b2dull << 16;
+template <int G> __device__ __forceinline__ __amdgpu_buffer_rsrc_t ws_rows(const DecodeArgs& a, int b, int h) {
+  return __builtin_amdgcn_make_buffer_rsrc(a.ws_o + ((int64_t)b * a.hq + h * G) * a.n_parts * kHeadDim, 0,
+                                           G * a.n_parts * kHeadDim * 4, 0x00020000);
+}
+template <int G> __device__ __forceinline__ __amdgpu_buffer_rsrc_t ws_lses(const DecodeArgs& a, int b, int h) {
+  return __builtin_amdgcn_make_buffer_rsrc(a.ws_lse + ((int64_t)b * a.hq + h * G) * a.n_parts, 0,
+                                           G * a.n_parts * 4, 0x00020000);
 }
 
 // NEW: the workgroup that holds the new token (the last one of the context)
@@ -590,11 +607,89 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
     if (np == 1) {
       store_out2<DT>(a.out, (int64_t)b * a.out_seq_stride + (int64_t)hq * kHeadDim + d2, o0 * inv,
                      o1 * inv);
-    } else {
+    } else if constexpr (NEW != kAppendMerge) {
       const int64_t slot = ((int64_t)b * a.hq + hq) * a.n_parts + part;
       *reinterpret_cast<float2*>(a.ws_o + slot * kHeadDim + d2) = make_float2(o0 * inv, o1 * inv);
       if (d2 == 0) a.ws_lse[slot] = mx + __log2f(L);
+    } else {
+      const u32x2 v = {__float_as_uint(o0 * inv), __float_as_uint(o1 * inv)};
+      __builtin_amdgcn_raw_buffer_store_b64(v, ws_rows<G>(a, b, h), ((g * a.n_parts + part) * kHeadDim + d2) * 4, 0, kSc1);
+      if (d2 == 0)
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(mx + __log2f(L)), ws_lses<G>(a, b, h),
+                                              (g * a.n_parts + part) * 4, 0, kSc1);
     }
+  }
+  if constexpr (NEW != kAppendMerge) return;
+  if (np == 1) return;
+
+  // The partition that finishes last combines them all, in partition order
+  // whichever it is.  Partial results are written and read past the XCDs' L2s
+  // (sc1, as the compiler's agent-scope atomics are), every lane waits for its
+  // own before the workgroup counts itself, and nothing waits for another
+  // workgroup.  A counter holds kCntTag in its upper 48 bits from its first
+  // use on (a workspace comes as it is) and goes back to zero finished.
+  __shared__ int s_last;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0) {
+    unsigned long long* cnt = a.ws_cnt + (int64_t)b * a.hkv + h;
+    unsigned long long v = __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if ((v & ~0xffffull) != kCntTag)
+      __hip_atomic_compare_exchange_strong(cnt, &v, kCntTag, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+    v = __hip_atomic_fetch_add(cnt, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_last = (int)(v & 0xffff) == np - 1;
+    if (s_last) __hip_atomic_store(cnt, kCntTag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (!s_last) return;
+  const __amdgpu_buffer_rsrc_t rows = ws_rows<G>(a, b, h), lses = ws_lses<G>(a, b, h);
+  // wave w: head g, partitions c, c + C, ...; lane: two dims
+  constexpr int C = G >= 4 ? 1 : 4 / G;
+  __shared__ float sm_w[C][G];
+  __shared__ float2 sm_o[C][G][64];
+#pragma unroll
+  for (int k = 0; k < (G > 4 ? G / 4 : 1); ++k) {
+    const int g = G >= 4 ? wave + 4 * k : wave % G, c = G >= 4 ? 0 : wave / G;
+    float mx = -INFINITY;
+    for (int p = lane; p < np; p += 64)
+      mx = fmaxf(mx, __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(lses, (g * a.n_parts + p) * 4, 0, kSc1)));
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    constexpr int V = 8;  // partitions in flight
+    float W = 0.f, o0 = 0.f, o1 = 0.f;
+    for (int p0 = c; p0 < np; p0 += V * C) {
+      u32 ls[V];
+      u32x2 ov[V];
+#pragma unroll
+      for (int u = 0; u < V; ++u) {
+        const int i = g * a.n_parts + min(p0 + u * C, np - 1);
+        ls[u] = __builtin_amdgcn_raw_buffer_load_b32(lses, i * 4, 0, kSc1);
+        ov[u] = __builtin_amdgcn_raw_buffer_load_b64(rows, (i * kHeadDim + 2 * lane) * 4, 0, kSc1);
+      }
+#pragma unroll
+      for (int u = 0; u < V; ++u) {
+        const float w = p0 + u * C < np ? fast_exp2(__uint_as_float(ls[u]) - mx) : 0.f;
+        W += w;
+        o0 = fmaf(w, __uint_as_float(ov[u][0]), o0);
+        o1 = fmaf(w, __uint_as_float(ov[u][1]), o1);
+      }
+    }
+    if constexpr (C > 1) {
+      if (lane == 0) sm_w[c][g] = W;
+      sm_o[c][g][lane] = make_float2(o0, o1);
+      __syncthreads();
+      if (c) return;
+#pragma unroll
+      for (int j = 1; j < C; ++j) {
+        W += sm_w[j][g];
+        o0 += sm_o[j][g][lane].x;
+        o1 += sm_o[j][g][lane].y;
+      }
+    }
+    const float inv = 1.f / W;
+    store_out2<DT>(a.out, (int64_t)b * a.out_seq_stride + (int64_t)(h * G + g) * kHeadDim + 2 * lane,
+                   o0 * inv, o1 * inv);
   }
 }
 
@@ -719,12 +814,14 @@ static void launch_decode_t(const DecodeArgs& a, hipStream_t s) {
   constexpr int U = DT == Dt::FP32 ? 4 : 8;
   if (a.qw) {
     if constexpr (DT != Dt::FP32) launch_decode_p<DT, G, U, kQkv>(a, s);
+  } else if (a.ws_cnt) {
+    launch_decode_p<DT, G, U, kAppendMerge>(a, s);
   } else if (a.k_new) {
     launch_decode_p<DT, G, U, kAppend>(a, s);
   } else {
     launch_decode_p<DT, G, U, kNone>(a, s);
   }
-  if (a.n_parts > 1)
+  if (a.n_parts > 1 && a.ws_cnt == nullptr)
     hipLaunchKernelGGL((decode_reduce_kernel<DT>), dim3(a.hq, a.n_seqs), dim3(256), 0, s, a);
 }
 
@@ -831,15 +928,31 @@ static int decode_common(const void* q, int64_t q_seq_stride, const void* k_cach
     a.bs_magic = 0;
     a.bs_mshift = 0;
   }
-  // length order only without a split: split partitions are already
-  // uniform work units, and the ordering costs every workgroup a few barriers
-  a.lpt = plan.n_parts == 1 && n_seqs >= 2 && n_seqs <= kLptMaxSeqs;
+  // Length order only without a split (split partitions are already uniform
+  // work units), and not for contexts of a few iterations that are all resident
+  // at once: finding the order costs every workgroup some 1.7 us (8 sequences of
+  // 69-250 tokens 8.6 us with it, 6.9 without; 64 of 10-500 17.1 and 17.6, 100 of
+  // 100-2000 82.5 and 100.1).
+  a.lpt = plan.n_parts == 1 && n_seqs >= 2 && n_seqs <= kLptMaxSeqs &&
+          (plan.part_tokens > 256 || (int64_t)n_seqs * n_kv_heads > 1024);
   a.lpt_max = max_context_len > 0
                   ? max_context_len
                   : (int32_t)std::min<int64_t>((int64_t)max_blocks_per_seq * block_size, INT32_MAX);
   if (plan.ws_bytes) {
     a.ws_o = reinterpret_cast<float*>(workspace);
     a.ws_lse = a.ws_o + (size_t)n_seqs * n_q_heads * plan.n_parts * kHeadDim;
+    // Room for counters past the partial results: a small append call combines
+    // them in its launch.  Writes past the L2s, the counting and the second read
+    // take the GPU longer than a second launch from some 4 partitions on (24
+    // sequences in 9 partitions 29.9 us against 25.7), but a caller that launches
+    // each call itself is bound by its launches (fp32, 4 sequences in 8
+    // partitions: 15.3 us a call with the second launch, 13.5 without).  The room
+    // is the caller's choice.
+    const size_t cnt = (plan.ws_bytes + 15) / 16 * 16;
+    const int64_t items = (int64_t)n_seqs * n_kv_heads;
+    if (nt.k && !nt.qw && plan.n_parts <= 8 && items * plan.n_parts <= 512 &&
+        workspace_bytes >= cnt + (size_t)items * 8)
+      a.ws_cnt = reinterpret_cast<unsigned long long*>((char*)workspace + cnt);
   }
   a.k_new = nt.k;
   a.v_new = nt.v;
@@ -928,7 +1041,7 @@ extern "C" int aac_decode_paged_noalloc(const void* q, int64_t q_seq_stride, con
   return decode_common(q, q_seq_stride, k_cache, v_cache, num_blocks, block_size, block_tables,
                        max_blocks_per_seq, context_lens, 0, n_seqs, max_context_len, n_q_heads,
                        n_kv_heads, head_dim, scale, out, out_seq_stride, ws,
-                       need ? (size_t)AAC_DECODE_SCRATCH_BYTES : 0, partition_tokens, dtype,
+                       need, partition_tokens, dtype,
                        (hipStream_t)stream);
 }
 

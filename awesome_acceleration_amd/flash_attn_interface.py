@@ -510,7 +510,13 @@ def flash_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, rotary_cos=None
         part = max(1, math.ceil(cap / int(num_splits)))
     L = _lib.lib()
     ws_bytes = _decode_ws_bytes(B, Hq, hkv, D, bs, mb, mcl, part)
-    wsp = _workspace(ws_bytes, q.device).data_ptr() if ws_bytes else None
+    wsp = None
+    if ws_bytes:
+        # an eager append of few sequences is bound by its launches: with room for
+        # counters one launch also combines the partitions
+        if k is not None and B * hkv <= 128 and not torch.cuda.is_current_stream_capturing():
+            ws_bytes = (ws_bytes + 15) // 16 * 16 + B * hkv * 8
+        wsp = _workspace(ws_bytes, q.device).data_ptr()
     if k is None:
         rc = L.aac_decode_paged(
             q3.data_ptr(), q_stride, k_cache.data_ptr(), v_cache.data_ptr(), nblk, bs,

@@ -173,7 +173,10 @@ int aac_prefill_varlen_store(const void* q, const void* k, const void* v, int64_
  * Bytes of split-K workspace aac_decode_paged needs for this shape.
  * max_context_len <= 0 means "table capacity" (max_blocks_per_seq *
  * block_size), partition_tokens <= 0 means "library's choice".  Returns 0
- * when the chosen plan needs no workspace.
+ * when the chosen plan needs no workspace.  A workspace_bytes larger by 8 bytes
+ * per (sequence, KV head) past this size rounded up to 16 lets a small append call
+ * combine its partitions in the attention launch instead of a second one; the
+ * workspace needs no initialisation, and a call uses no more of it than that.
  */
 size_t aac_decode_workspace_bytes(int32_t n_seqs, int32_t n_q_heads, int32_t n_kv_heads,
                                   int32_t head_dim, int32_t block_size, int32_t max_blocks_per_seq,
