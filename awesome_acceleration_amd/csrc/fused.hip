@@ -140,8 +140,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_tok_kernel(QkArgs a) {
     u32x4 xr[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int hh = h0 + 4 * u + r;
-      if (hh < heads) xr[u] = get16<NT>(src + (int64_t)hh * kHeadDimFused);
+      const int hh = min(h0 + 4 * u + r, heads - 1);  // no branch between the loads
+      xr[u] = get16<NT>(src + hh * kHeadDimFused);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {

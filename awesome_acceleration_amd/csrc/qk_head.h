@@ -45,12 +45,18 @@ __device__ __forceinline__ u32x4 pack8(const float* f) {
   return w;
 }
 
-// Both values rounded to the activation type: one convert and two unpacks.
+// Both values rounded to the activation type: bf16 has a convert of pairs (and
+// two unpacks), fp16 converts one by one.
 template <Dt DT>
 __device__ __forceinline__ void round2(float& a, float& b) {
-  const u32 w = Cvt<DT>::pack(a, b);
-  a = Cvt<DT>::lo(w);
-  b = Cvt<DT>::hi(w);
+  if constexpr (DT == Dt::BF16) {
+    const u32 w = Cvt<DT>::pack(a, b);
+    a = Cvt<DT>::lo(w);
+    b = Cvt<DT>::hi(w);
+  } else {
+    a = Cvt<DT>::round(a);
+    b = Cvt<DT>::round(b);
+  }
 }
 
 // 16 bytes to memory; NT: non-temporal, past the caches.
@@ -183,13 +189,13 @@ __device__ __forceinline__ void norm_rope_head(const QkArgs& a, int64_t t, int h
   }
 }
 
-// sin of the lane's dims, negated in the first half: rounding is symmetric,
-// so (-partner) * sin and partner * (-sin) are the same bits.
+// sin of the lane's dims, negated in the first half (a sign bit per packed value:
+// as fp16 the products then still fold into half-precision operations): rounding
+// is symmetric, so (-partner) * sin and partner * (-sin) are the same bits.
 template <Dt DT>
 __device__ __forceinline__ void signed_sin(const u32x4& sin8, int li, float* sf) {
-  unpack8<DT>(sin8, sf);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) sf[i] = li < 8 ? -sf[i] : sf[i];
+  const u32 sign = li < 8 ? 0x80008000u : 0u;
+  unpack8<DT>(u32x4{sin8[0] ^ sign, sin8[1] ^ sign, sin8[2] ^ sign, sin8[3] ^ sign}, sf);
 }
 template <Dt DT>
 __device__ __forceinline__ void signed_sin(const u16* sin8, int li, float* sf) {
