@@ -33,8 +33,8 @@ Also reported on the same line:
                 and torch's own flash attention (SDPA, flash backend) on the
                 same shape for reference;
   prefill_one_request  one 2048-token request: too few work items for the
-                CUs, so each item's key range is split over two workgroups
-                (the same call unsplit beside it);
+                CUs, so the keys are split over a workgroup's waves (the
+                same call without a workspace beside it);
   prefill_long  the same kernel on 8 x 8192 causal tokens: its steady-state
                 rate, where per-item start and epilogue costs are small;
   prefill_engine  the prefill call the engine makes for 256 fresh 1024-token
@@ -570,9 +570,9 @@ def bench_prefill_engine(torch, fai, paged, dev, args, nseq=256, L=1024, hq=16, 
 
 
 def bench_prefill_one_request(torch, fai, dev, args, L=2048, hq=16, hkv=8):
-    """One 2048-token request (16/8 heads, causal): 128 work items for 256
-    CUs, so each item's key range is split over two workgroups and merged;
-    the same call without the split (no workspace) beside it."""
+    """One 2048-token request (16/8 heads, causal), on the kernel that splits
+    the keys over a workgroup's waves; the same call without a workspace
+    beside it (``us_unsplit``: this kernel needs none)."""
     from awesome_acceleration_amd import _lib
     d = 128
     g = torch.Generator(device=dev).manual_seed(args.seed)
@@ -600,7 +600,7 @@ def bench_prefill_one_request(torch, fai, dev, args, L=2048, hq=16, hkv=8):
     t0 = launch_avg(torch, unsplit, args.steps)
     ws = lib.aac_prefill_workspace_bytes(1, L, L, hq, hkv, d, 1)
     return {"workload": f"varlen causal prefill of one {L}-token request, {hq}/{hkv} heads, "
-                        "head_dim 128, bf16: key ranges split over two workgroups and merged",
+                        "head_dim 128, bf16: keys split over each workgroup's waves",
             "us_attend": round(t * 1e6, 2), "us_unsplit": round(t0 * 1e6, 2),
             "workspace_bytes": int(ws),
             "roofline": {"bound": "mfma", "achieved": round(flops / t / 1e12, 2),
