@@ -666,7 +666,9 @@ static int launch_g(const Args& a, int g, int max_q, int n_cu, hipStream_t st) {
 // 1 x 4096 111.9 -> 92.0; not split because it measured slower: 256 items
 // of at most 16 tiles (8 x 1024 at 8/4 heads 34.8 -> 43.0, 4 x 1024 at 16/8
 // 34.0 -> 43.3), items under 16 tiles (1 x 512 19.0 -> 19.4, 2 x 256
-// 12.3 -> 15.9); four pieces never beat two by more than noise.
+// 12.3 -> 15.9); four pieces never beat two by more than noise.  Calls with groups
+// of 2, 4 and 8 that this plan would split run on prefill_split.hip instead (1 x
+// 1024 at 16/8 heads 14.5 us, 1 x 2048 29.2); it serves group 1.
 struct SplitPlan {
   int32_t n_split;
   int64_t n_items;  // items (without pieces): counters in the workspace
