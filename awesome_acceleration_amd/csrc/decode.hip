@@ -38,17 +38,16 @@
 //   type and P.V is v_dot2 over V words paired across two tokens (v_perm);
 //   fp32: unpacked fp32 FMAs with q pre-scaled.  The 16 row states of a workgroup are
 //   merged at the end (cross-row shuffles inside a wave, LDS across waves).
+//   A sequence whose context spans one partition writes the final output
+//   directly; longer contexts write a normalised partial output and its
+//   log-sum-exp to the workspace, and a second kernel combines the
+//   partitions (the FlashDecoding split-K method).
 //
 // The new token (aac_decode_append_paged, aac_decode_qkv_paged): appended by
 // the attention launch itself, see NEW at the kernel.  Against a store launch
 // before it: 24 slot-layout sequences of 100-2063 tokens 29.5 -> 26.5 us a call, a
 // 28-layer step of 4 sequences 935 -> 881 (with the q/k norm + RoPE folded in
 // too); 256 x 1-2k the same (240.8 and 240.9).
-//
-//   A sequence whose context spans one partition writes the final output
-//   directly; longer contexts write a normalised partial output and its
-//   log-sum-exp to the workspace, and a second kernel combines the
-//   partitions (the FlashDecoding split-K method).
 //
 // Bytes per launch (the HBM roofline): every context token's K and V row of
 // each KV head is read exactly once, 2 * Hkv * D * elem_bytes per token, plus
