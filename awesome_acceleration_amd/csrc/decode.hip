@@ -45,9 +45,10 @@
 //
 // The new token (aac_decode_append_paged, aac_decode_qkv_paged): appended by
 // the attention launch itself, see NEW at the kernel.  Against a store launch
-// before it: 24 slot-layout sequences of 100-2063 tokens 29.5 -> 26.5 us a call, a
-// 28-layer step of 4 sequences 935 -> 881 (with the q/k norm + RoPE folded in
-// too); 256 x 1-2k the same (240.8 and 240.9).
+// before it: 24 slot-layout sequences of 100-2063 tokens 27.1 -> 25.6 us (graph
+// replay), a 28-layer step of 4 sequences some 40 us less with the q/k norm + RoPE
+// folded in too.  The search for rows that share blocks is 0.3-1.2 us of that a
+// launch (without it 24.4; the step 824 against 838).
 //
 // Bytes per launch (the HBM roofline): every context token's K and V row of
 // each KV head is read exactly once, 2 * Hkv * D * elem_bytes per token, plus
@@ -148,15 +149,16 @@ template <Dt DT> struct Raw8 {
   }
 };
 
-__device__ __forceinline__ int context_len(const DecodeArgs& a, int b) {
-  int ctx = a.lens[b] + a.lens_add;
+__device__ __forceinline__ int clip_len(const DecodeArgs& a, int len) {
+  int ctx = len + a.lens_add;
   const int cap = a.max_blocks * a.block_size;
   ctx = ctx < 0 ? 0 : ctx;
   return ctx > cap ? cap : ctx;
 }
+__device__ __forceinline__ int context_len(const DecodeArgs& a, int b) { return clip_len(a, a.lens[b]); }
 
 __device__ __forceinline__ int parts_of(const DecodeArgs& a, int ctx) {
-  int n = (int)cdiv(ctx, a.part_tokens);
+  const int n = (int)(((uint32_t)ctx + (uint32_t)a.part_tokens - 1) / (uint32_t)a.part_tokens);
   return n > a.n_parts ? a.n_parts : n;
 }
 
@@ -249,10 +251,32 @@ template <int G> __device__ __forceinline__ __amdgpu_buffer_rsrc_t ws_lses(const
                                            G * a.n_parts * 4, 0x00020000);
 }
 
+// One dword per lane from global memory straight into LDS at p + lane.  Inline
+// assembly: the compiler neither moves the load (it sinks ordinary ones to their
+// first use, behind the wait for the context length) nor waits for it; read p
+// behind landed().
+__device__ __forceinline__ void to_lds4(const int32_t* src, int* p) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
+               :
+               : "v"(src), "s"((u32)(uintptr_t)(__attribute__((address_space(3))) int*)p)
+               : "memory", "m0");
+#pragma clang diagnostic pop
+}
+__device__ __forceinline__ void landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // NEW: the workgroup that holds the new token (the last one of the context)
 // starts its online softmax from it, straight from the given rows, and writes
 // them to the caches: the loop is that of kNone, and there is no launch before
-// this one.
+// this one.  The result is that of a store launch before the attention also
+// where rows of the call share blocks (one sequence given as several rows, at
+// positions n, n + 1, ...): in a workgroup whose tokens include another row's new
+// one, each wave first writes that row to the cache too, the same bytes as its
+// owner, and reads what it wrote.  Looked for before the loop: beside its first
+// loads, or behind it with a second pass, the search's registers spilled or its
+// code cost more than the latency (step of 4 sequences 857 us, and 833-850 with the
+// tables scanned entry by entry, whose cost grows with them: 64 x 10-500 21 us).
 template <Dt DT, int G, int U, bool POW2, int NEW>
 // Occupancy: with G <= 2 the kernel fits 128 VGPRs, i.e. four workgroups per
 // CU (16 wavefronts); larger groups hold more accumulators.
@@ -274,7 +298,7 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
   const int b = a.lpt ? __builtin_amdgcn_readfirstlane(seq_of_rank(a, blockIdx.z, tid))
                      : (int)blockIdx.z;  // wave-uniform (SGPR) either way
   constexpr int R = 16;  // token rows of the workgroup (one per DPP row)
-  const int lane = tid & 63, wave = tid >> 6;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, grp = lane >> 4;
   const int rslot = wave * 4 + grp;  // 0 .. R - 1
   const int t0 = part * a.part_tokens;
@@ -290,6 +314,7 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
   // and the query rows.  The first K/V loads then wait for one load, not four,
   // and the query's preparation runs while they are in flight (28-layer step of
   // 4 sequences 879 -> 870 us; 256 x 1-2k 241.2 -> 240.2, 64 x 16k-32k 989.5 -> 984.5).
+  const int len = a.lens[b];
   int blk[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) blk[u] = bt[min(block_index(t0 + rslot + R * u), a.max_blocks - 1)];
@@ -302,29 +327,44 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
     for (int g = 0; g < G; ++g) qr[g].load(qb + (int64_t)g * kHeadDim * ES);
   }
   // NEW == kQkv: the norm weight and RoPE rows of the query heads
-  u32x4 wraw, craw, sraw;
-  int64_t rope = 0;
-  if constexpr (NEW == kQkv) {
-    const int pos = a.positions[b];
-    rope = (int64_t)(pos < 0 ? 0 : (pos >= a.max_pos ? a.max_pos - 1 : pos)) * kHeadDim + li * 8;
-    wraw = *reinterpret_cast<const u32x4*>(a.qw + li * 8);
-    craw = *reinterpret_cast<const u32x4*>(a.cos + rope);
-    sraw = *reinterpret_cast<const u32x4*>(a.sin + rope);
+  struct Rope {
+    u32x4 c, s;
+  };
+  auto rope_of = [&](int row) {
+    Rope r = {};
+    if constexpr (NEW == kQkv) {
+      const int64_t at = (int64_t)min(max(a.positions[row], 0), a.max_pos - 1) * kHeadDim + li * 8;
+      r.c = *reinterpret_cast<const u32x4*>(a.cos + at);
+      r.s = *reinterpret_cast<const u32x4*>(a.sin + at);
+    }
+    return r;
+  };
+  const Rope rope = rope_of(b);
+  u32x4 wraw;
+  if constexpr (NEW == kQkv) wraw = *reinterpret_cast<const u32x4*>(a.qw + li * 8);
+  // NEW: wave 3 looks for rows that share blocks (below), from the positions of the
+  // call's first 64 rows and the first 64 blocks of this partition.  One wave, as at
+  // the start all waves of a CU compete for issue.
+  __shared__ int s_new[NEW == kNone ? 1 : 2][64];
+  __shared__ int s_share;
+  if (NEW != kNone && wave == 3) {
+    to_lds4(a.lens + min(lane, a.n_seqs - 1), s_new[0]);
+    to_lds4(bt + min(block_index(t0) + lane, a.max_blocks - 1), s_new[1]);
   }
   // RMSNorm + RoPE of one head row
-  auto new_head = [&](const u32x4& raw, const u32x4& w) {
+  auto new_head = [&](const u32x4& raw, const u32x4& w, const Rope& r) {
     u32x4 o = raw;
     if constexpr (NEW == kQkv) {
       float wf[8], cf[8], sf[8];
       fz::unpack8<DT>(w, wf);
-      fz::unpack8<DT>(craw, cf);
-      fz::signed_sin<DT>(sraw, li, sf);
+      fz::unpack8<DT>(r.c, cf);
+      fz::signed_sin<DT>(r.s, li, sf);
       o = fz::norm_rope_row<DT>(raw, a.eps, wf, cf, sf);
     }
     return o;
   };
 
-  const int ctx = context_len(a, b);
+  const int ctx = clip_len(a, len);
   const int np = parts_of(a, ctx);
   if (part >= np) {
     if (part == 0) {  // empty context: zeros (FA2 convention)
@@ -334,11 +374,12 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
                        0.f, 0.f);
       }
     }
+    if constexpr (NEW != kNone) landed();
     return;
   }
   // NEW: the last partition takes the new token (position lens[b], unless that
   // lies outside the table) apart from the loop, which ends before it.
-  const bool has_new = NEW != kNone && part == np - 1 && a.lens[b] == ctx - 1;
+  const bool has_new = NEW != kNone && part == np - 1 && len == ctx - 1;
   const int t1 = (part == np - 1) ? ctx - (has_new ? 1 : 0) : t0 + a.part_tokens;
 
   const int64_t tok_bytes = (int64_t)a.hkv * kHeadDim * ES;  // cache row stride
@@ -373,7 +414,7 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
   auto prepare = [&]() {
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-      if constexpr (NEW == kQkv) qr[g].w[0] = new_head(qr[g].w[0], wraw);
+      if constexpr (NEW == kQkv) qr[g].w[0] = new_head(qr[g].w[0], wraw, rope);
       if constexpr (PK) {
 #pragma unroll
         for (int w = 0; w < 4; ++w) qp[g][w] = qr[g].w[0][w];
@@ -396,6 +437,65 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
   bool ready = kQueryFirst;
   if constexpr (kQueryFirst) prepare();
 
+  // The rows r0 .. r0 + 63 whose new token is one of [t0, t1), as a lane mask, with
+  // their positions and blocks: rows in lanes, the partition's blocks one by one.
+  // From memory, or the first ones from LDS.
+  struct New {
+    int pos, blk;
+  };
+  auto shared_rows = [&](int r0, bool lds, New& e) {
+    const int row = min(r0 + lane, a.n_seqs - 1);
+    e.pos = lds ? s_new[0][lane] : a.lens[row];
+    const int bi = block_index(max(e.pos, 0)), off = e.pos - bi * a.block_size;
+    e.blk = a.block_tables[(int64_t)row * a.max_blocks + min(bi, a.max_blocks - 1)];
+    bool hit = false;
+    if (t1 > t0) {
+      const int first = block_index(t0), last = block_index(t1 - 1);
+      for (int i0 = first; i0 <= last; i0 += 64) {
+        const int own = lds && i0 == first ? s_new[1][lane] : bt[min(i0 + lane, a.max_blocks - 1)];
+        const int n = min(64, last + 1 - i0);
+        for (int j = 0; j < n; ++j) {
+          const int t = (i0 + j) * a.block_size + off;
+          hit |= __builtin_amdgcn_readlane(own, j) == e.blk && t >= t0 && t < t1;
+        }
+      }
+    }
+    // the row's new token is inside the table, its block inside the cache
+    return __ballot(hit && r0 + lane < a.n_seqs && e.pos >= 0 && bi < a.max_blocks && (uint32_t)e.blk < nb32);
+  };
+  // Write those rows to the caches (every wave for itself).
+  auto settle = [&]() {
+    for (int r0 = 0; r0 < a.n_seqs; r0 += 64) {
+      New e;
+      for (unsigned long long rows = shared_rows(r0, false, e); rows; rows &= rows - 1) {
+        const int i = __ffsll(rows) - 1, row = r0 + i;
+        const int64_t to = row_off(__builtin_amdgcn_readlane(e.pos, i), __builtin_amdgcn_readlane(e.blk, i));
+        const int64_t hd = (int64_t)h * kHeadDim + li * 8;
+        Raw8<DT> kx, vx;
+        kx.load(reinterpret_cast<const char*>(a.k_new) + (row * a.k_new_stride + hd) * ES);
+        vx.load(reinterpret_cast<const char*>(a.v_new) + (row * a.v_new_stride + hd) * ES);
+        if constexpr (NEW == kQkv)
+          kx.w[0] = new_head(kx.w[0], *reinterpret_cast<const u32x4*>(a.kw + li * 8), rope_of(row));
+        if (lane < kRowLanes) {
+          kx.store(const_cast<char*>(kbase) + to);
+          vx.store(const_cast<char*>(vbase) + to);
+        }
+      }
+    }
+    landed();
+  };
+  if constexpr (NEW != kNone) {
+    if (wave == 3) {
+      landed();
+      unsigned long long rows = 0;
+      New e;
+      for (int r0 = 0; r0 < a.n_seqs; r0 += 64) rows |= shared_rows(r0, r0 == 0, e);
+      if (lane == 0) s_share = rows != 0;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (s_share) settle();
+  }
+
   // The new token: row 0 of the workgroup starts its online softmax from the
   // given rows and writes them to the caches (not to a block outside the
   // cache: then the row that a bad entry reads takes their place).
@@ -412,7 +512,7 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
     kx.load(store ? reinterpret_cast<const char*>(a.k_new) + (b * a.k_new_stride + hd) * ES : kbase + off);
     vx.load(store ? reinterpret_cast<const char*>(a.v_new) + (b * a.v_new_stride + hd) * ES : vbase + off);
     if constexpr (NEW == kQkv) {
-      if (store) kx.w[0] = new_head(kx.w[0], *reinterpret_cast<const u32x4*>(a.kw + li * 8));
+      if (store) kx.w[0] = new_head(kx.w[0], *reinterpret_cast<const u32x4*>(a.kw + li * 8), rope);
     }
     float vf[8], kf[PK ? 1 : 8];
     vx.unpack(vf);
@@ -1056,10 +1156,13 @@ extern "C" int aac_decode_append_paged(const void* q, int64_t q_seq_stride, cons
                                        int32_t dtype, void* stream) {
   if (head_dim != kHeadDim) return AAC_ERR_UNSUPPORTED;
   // The append runs inside the attention launch when its rows suit the 16-byte
-  // loads there; anything else takes the general append first.
+  // loads there and there are at most 64 of them, a lane each in the search for
+  // shared blocks; anything else takes the general append first (graph replay, one
+  // launch against two, us: 24 x 100-2063 25.6 and 27.1, 64 x 10-500 16.0 and 17.4,
+  // 1 x 20,000 at 32/8 heads 24.7 and 25.9; 256 x 1-2k 249.5 and 245.3).
   const int es = dtype == AAC_DTYPE_FP32 ? 4 : 2;
   const int g = n_kv_heads > 0 && n_q_heads > 0 && n_q_heads % n_kv_heads == 0 ? n_q_heads / n_kv_heads : 0;
-  if (n_seqs > 0 && (g == 1 || g == 2 || g == 4 || g == 8) && k && v && k_cache && v_cache &&
+  if (n_seqs > 0 && n_seqs <= 64 && (g == 1 || g == 2 || g == 4 || g == 8) && k && v && k_cache && v_cache &&
       block_tables && cache_seqlens && num_blocks > 0 && k_tok_stride >= (int64_t)n_kv_heads * head_dim &&
       v_tok_stride >= (int64_t)n_kv_heads * head_dim && ((uintptr_t)k | (uintptr_t)v) % 16 == 0 &&
       (k_tok_stride * es) % 16 == 0 && (v_tok_stride * es) % 16 == 0) {

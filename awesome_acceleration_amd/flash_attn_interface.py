@@ -382,7 +382,8 @@ def decode_qkv_paged(qkv, n_q_heads, q_norm_weight, k_norm_weight, eps, cos, sin
     ``qkv [B, (Hq + 2 Hkv) * D]``: q/k RMSNorm + RoPE at ``positions``, the
     append at ``cache_seqlens`` and the attention over ``cache_seqlens + 1``
     tokens (model/model.py:219-240) in one launch (and the reduction of a
-    split).  Returns ``[B, Hq, D]``; bf16 and fp16."""
+    split); rows may share blocks as in ``flash_attn_with_kvcache``.  Returns
+    ``[B, Hq, D]``; bf16 and fp16."""
     _on_gpu(qkv, q_norm_weight, k_norm_weight, cos, sin, positions, k_cache, v_cache, block_tables,
             cache_seqlens)
     _require(qkv.dim() == 2 and qkv.stride(1) == 1, "qkv must be [B, width]")
@@ -452,7 +453,9 @@ def flash_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, rotary_cos=None
     ``[num_blocks, block_size, Hkv, D]``.  When ``k``/``v`` (``[B, 1, Hkv,
     D]``) are given they are written at position ``cache_seqlens[b]`` first
     and the call attends over ``cache_seqlens[b] + 1`` tokens, otherwise over
-    ``cache_seqlens[b]``.  ``cache_seqlens`` is not modified.  Returns a new
+    ``cache_seqlens[b]``.  All rows are written before any is read: one
+    sequence may be given as several rows (the same table, positions ``n``,
+    ``n + 1``, ...).  ``cache_seqlens`` is not modified.  Returns a new
     ``[B, 1, Hq, D]`` tensor.
     """
     if softcap or alibi_slopes is not None or window_size != (-1, -1):

@@ -240,8 +240,11 @@ int aac_decode_paged_noalloc(const void* q, int64_t q_seq_stride, const void* k_
  * cache_seqlens[b] (aac_kv_append_paged), then attend over
  * cache_seqlens[b] + 1 tokens.  cache_seqlens is not modified.
  * max_context_len bounds cache_seqlens[b] + 1 (<= 0: table capacity).
- * The append runs inside the attention launch: as in flash_attn, sequences of
- * one call do not see each other's new tokens in a shared block.
+ * The append runs inside the attention launch with the result of an append
+ * before it: every row of the call sees the new tokens of all rows in blocks that
+ * its table shares with them (one sequence given as several rows, at positions n,
+ * n + 1, ...).  Two rows that write the same cache row: one of them stays in the
+ * cache.
  * Replaces model/model.py:233-240.
  */
 int aac_decode_append_paged(const void* q, int64_t q_seq_stride, const void* k, const void* v,
@@ -260,6 +263,7 @@ int aac_decode_append_paged(const void* q, int64_t q_seq_stride, const void* k, 
  * positions[b] (model/model.py:219-228, as aac_qk_norm_rope_store), the append
  * of k and v at cache_seqlens[b], and the attention over cache_seqlens[b] + 1
  * tokens (model/model.py:233-240), without the normalised q and k in memory.
+ * Rows that share blocks see each other's new tokens, as above.
  * dtype bf16 or fp16; the workspace is aac_decode_workspace_bytes'.
  */
 int aac_decode_qkv_paged(const void* qkv, int64_t qkv_row_stride, const void* q_norm_weight,

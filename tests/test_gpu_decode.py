@@ -452,3 +452,88 @@ def test_decode_from_projection_rows(gpu, dtype, hq, hkv, bs):
     torch.cuda.synchronize()
     assert torch.equal(kc, kc2) and torch.equal(vc, vc2)
     _close_decode(out, ref, dtype, float(vc2.float().abs().max()))
+
+
+def _shared_rows(gpu, dtype, hkv, bs, n, seed):
+    """Rows that share blocks with each other: n rows of one sequence at
+    successive positions that cross a block, two sequences with a common prefix,
+    and a row that has another row's new block early in its table; every row to
+    be written holds NaN."""
+    g = torch.Generator(device=gpu).manual_seed(seed)
+    W = 4 + -(-n // bs)
+    pool = 3 * W + 3 * (n + 4)
+    perm = torch.randperm(pool, generator=g, device=gpu).to(torch.int32).tolist()
+    one, a, b = perm[:W], perm[W:2 * W], perm[2 * W:3 * W]
+    first = bs - 2
+    rows = [one] * n + [a, a[:1] + b[1:]]
+    lens = [first + i for i in range(n)] + [2 * bs + 1, bs + 3]
+    rows.append([a[2], b[0]] + perm[3 * W:4 * W - 2])  # block a[2] takes row n's new token
+    lens.append(bs + 5)
+    order = torch.randperm(len(rows), generator=g, device=gpu).tolist()
+    rows, lens = [rows[i] for i in order], [lens[i] for i in order]
+    bt = torch.tensor(rows, dtype=torch.int32, device=gpu)
+    sl = torch.tensor(lens, dtype=torch.int32, device=gpu)
+    kc = torch.randn((pool, bs, hkv, 128), generator=g, device=gpu).to(dtype)
+    vc = torch.randn((pool, bs, hkv, 128), generator=g, device=gpu).to(dtype)
+    slots = torch.tensor([r[p // bs] * bs + p % bs for r, p in zip(rows, lens)], device=gpu)
+    vc.view(-1, hkv, 128)[slots] = float("nan")
+    return g, kc, vc, bt, sl, slots
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("hq,hkv,bs,n", [(16, 8, 64, 3), (32, 8, 100, 9), (8, 8, 16, 70), (16, 2, 256, 12)])
+def test_append_rows_that_share_blocks(gpu, dtype, hq, hkv, bs, n):
+    """All rows of an append call are stored before any is attended: rows of one
+    sequence see their predecessors' new tokens, in any order of the rows."""
+    print(f"case: append with shared blocks {dtype} {hq}/{hkv} block {bs} rows {n}", flush=True)
+    g, kc0, vc0, bt, sl, slots = _shared_rows(gpu, dtype, hkv, bs, n, 14)
+    B = sl.shape[0]
+    q = torch.randn((B, 1, hq, 128), generator=g, device=gpu).to(dtype)
+    k = torch.randn((B, 1, hkv, 128), generator=g, device=gpu).to(dtype)
+    v = torch.randn((B, 1, hkv, 128), generator=g, device=gpu).to(dtype)
+    kc2, vc2 = kc0.clone(), vc0.clone()
+    kc2.view(-1, hkv, 128)[slots], vc2.view(-1, hkv, 128)[slots] = k[:, 0], v[:, 0]
+    for splits in (0, 4):
+        kc, vc = kc0.clone(), vc0.clone()
+        out = fai.flash_attn_with_kvcache(q, kc, vc, k=k, v=v, cache_seqlens=sl, block_table=bt,
+                                          num_splits=splits)
+        ref = fai.flash_attn_with_kvcache(q, kc2, vc2, cache_seqlens=sl + 1, block_table=bt,
+                                          num_splits=splits)
+        torch.cuda.synchronize()
+        _close_decode(out, ref, dtype, float(vc2.float().abs().max()))
+        assert torch.equal(kc, kc2) and torch.equal(vc, vc2)
+    if dtype == torch.float32:
+        return
+    qkv = torch.randn((B, (hq + 2 * hkv) * 128), generator=g, device=gpu).to(dtype)
+    qw, kw = (1 + 0.3 * torch.randn((2, 128), generator=g, device=gpu)).to(dtype)
+    ang = torch.rand((300, 128), generator=g, device=gpu) * 6.28
+    cos, sin = ang.cos().to(dtype), ang.sin().to(dtype)
+    kc, vc, kc2, vc2 = kc0.clone(), vc0.clone(), kc0.clone(), vc0.clone()
+    q, _ = fz.qk_norm_rope_store(qkv, hq, hkv, qw, kw, 1e-6, cos, sin, sl, kc2, vc2,
+                                 block_tables=bt, cache_seqlens=sl, want_k=False)
+    ref = fai.decode_paged(q, kc2, vc2, bt, sl + 1)
+    out = fai.decode_qkv_paged(qkv, hq, qw, kw, 1e-6, cos, sin, sl, kc, vc, bt, sl)
+    torch.cuda.synchronize()
+    assert torch.equal(kc, kc2) and torch.equal(vc, vc2)
+    _close_decode(out, ref, dtype, float(vc2.float().abs().max()))
+
+
+def test_append_rows_of_one_slot(gpu):
+    """The slot layout: three rows of slot 1, the middle one between rows of
+    other slots."""
+    print("case: append rows of one slot", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(15)
+    idx = torch.tensor([1, 0, 1, 2, 1], dtype=torch.int32, device=gpu)
+    sl = torch.tensor([40, 7, 41, 0, 42], dtype=torch.int32, device=gpu)
+    kc = torch.randn((3, 300, 8, 128), generator=g, device=gpu).bfloat16()
+    vc = torch.randn((3, 300, 8, 128), generator=g, device=gpu).bfloat16()
+    q = torch.randn((5, 1, 16, 128), generator=g, device=gpu).bfloat16()
+    k, v = torch.randn((2, 5, 1, 8, 128), generator=g, device=gpu).bfloat16()
+    vc[idx.long(), sl.long()] = float("nan")
+    kc2, vc2 = kc.clone(), vc.clone()
+    kc2[idx.long(), sl.long()], vc2[idx.long(), sl.long()] = k[:, 0], v[:, 0]
+    out = fai.flash_attn_with_kvcache(q, kc, vc, k=k, v=v, cache_seqlens=sl, cache_batch_idx=idx)
+    ref = fai.flash_attn_with_kvcache(q, kc2, vc2, cache_seqlens=sl + 1, cache_batch_idx=idx)
+    torch.cuda.synchronize()
+    assert torch.equal(kc, kc2) and torch.equal(vc, vc2)
+    _close_decode(out, ref, torch.bfloat16, float(vc2.float().abs().max()))
