@@ -768,10 +768,12 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
       }
 #pragma unroll
       for (int u = 0; u < V; ++u) {
-        const float w = p0 + u * C < np ? fast_exp2(__uint_as_float(ls[u]) - mx) : 0.f;
-        W += w;
-        o0 = fmaf(w, __uint_as_float(ov[u][0]), o0);
-        o1 = fmaf(w, __uint_as_float(ov[u][1]), o1);
+        // past the end: nothing, not 0 x the last partition's (infinite?) result
+        const bool in = p0 + u * C < np;
+        const float w = fast_exp2(__uint_as_float(ls[u]) - mx);
+        W += in ? w : 0.f;
+        o0 = in ? fmaf(w, __uint_as_float(ov[u][0]), o0) : o0;
+        o1 = in ? fmaf(w, __uint_as_float(ov[u][1]), o1) : o1;
       }
     }
     if constexpr (C > 1) {
@@ -822,10 +824,12 @@ __global__ __launch_bounds__(256) void decode_reduce_kernel(DecodeArgs a) {
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const float w = p + 4 * u < np ? fast_exp2(lse[u] - mx) : 0.f;
-      W += w;
-      o0 = fmaf(w, o[u].x, o0);
-      o1 = fmaf(w, o[u].y, o1);
+      // past the end: nothing, not 0 x the last partition's (infinite?) result
+      const bool in = p + 4 * u < np;
+      const float w = fast_exp2(lse[u] - mx);
+      W += in ? w : 0.f;
+      o0 = in ? fmaf(w, o[u].x, o0) : o0;
+      o1 = in ? fmaf(w, o[u].y, o1) : o1;
     }
   }
   __shared__ float sw[4];

@@ -537,3 +537,34 @@ def test_append_rows_of_one_slot(gpu):
     torch.cuda.synchronize()
     assert torch.equal(kc, kc2) and torch.equal(vc, vc2)
     _close_decode(out, ref, torch.bfloat16, float(vc2.float().abs().max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("append", [False, True])
+@pytest.mark.parametrize("splits", [2, 5, 7, 8])
+def test_infinite_values_in_the_last_partition(gpu, dtype, append, splits):
+    """An infinite V element gives an infinite output, not NaN, however many
+    partitions the context is split in (the combination loads the last one again
+    past its end)."""
+    print(f"case: infinite values {dtype} append={append} splits={splits}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(16)
+    B, n = 2, 560
+    q = 0.1 * torch.randn((B, 1, 16, 128), generator=g, device=gpu)
+    q = q.to(dtype)
+    kc = torch.randn((B, n, 8, 128), generator=g, device=gpu).to(dtype)
+    vc = torch.randn((B, n, 8, 128), generator=g, device=gpu).to(dtype)
+    vc[0, n - 3, :, 5] = float("inf")
+    vc[1, n - 3, :, 6] = float("-inf")
+    kw = {}
+    if append:
+        kw = dict(k=kc[:, -1:].clone(), v=vc[:, -1:].clone())
+    out = fai.flash_attn_with_kvcache(q, kc, vc, cache_seqlens=n - 1 if append else n,
+                                      num_splits=splits, **kw)
+    torch.cuda.synchronize()
+    s = torch.einsum("bhgd,bnhd->bhgn", q.view(B, 8, 2, 128).double(), kc.double()) / 128 ** 0.5
+    ref = torch.einsum("bhgn,bnhd->bhgd", s.softmax(-1), vc.double().nan_to_num(0, 0, 0))
+    ref = ref.reshape(B, 1, 16, 128)
+    ref[0, ..., 5], ref[1, ..., 6] = float("inf"), float("-inf")
+    fin = ref.isfinite()
+    assert torch.equal(out[~fin].double(), ref[~fin])
+    _close_decode(out[fin], ref[fin], dtype, float(vc[vc.isfinite()].abs().max()))
