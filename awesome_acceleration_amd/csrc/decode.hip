@@ -151,9 +151,9 @@ template <Dt DT> struct Raw8 {
 
 __device__ __forceinline__ int clip_len(const DecodeArgs& a, int len) {
   int ctx = len + a.lens_add;
-  const int cap = a.max_blocks * a.block_size;
+  const int64_t cap = (int64_t)a.max_blocks * a.block_size;  // may lie past 2^31
   ctx = ctx < 0 ? 0 : ctx;
-  return ctx > cap ? cap : ctx;
+  return ctx > cap ? (int)cap : ctx;
 }
 __device__ __forceinline__ int context_len(const DecodeArgs& a, int b) { return clip_len(a, a.lens[b]); }
 
@@ -301,12 +301,14 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, grp = lane >> 4;
   const int rslot = wave * 4 + grp;  // 0 .. R - 1
-  const int t0 = part * a.part_tokens;
+  const int t0 = (int)((uint32_t)part * (uint32_t)a.part_tokens);  // past 2^31: no such partition
   const int32_t* bt = a.block_tables + (int64_t)b * a.max_blocks;
   const uint32_t nb32 = a.num_blocks < 0x7fffffff ? (uint32_t)a.num_blocks : 0x7fffffffu;
   auto block_index = [&](int t) {
     return POW2 ? t >> a.bs_shift : (int)(((uint64_t)(uint32_t)t * a.bs_magic) >> a.bs_mshift);
   };
+  // an entry of the row's table for any t, before it is known to be a token
+  auto entry = [&](int i) { return bt + min((uint32_t)i, (uint32_t)a.max_blocks - 1u); };
 
   // A call of few sequences is a chain of latencies, so everything that does not
   // depend on the context length is loaded beside it: the block numbers of the
@@ -317,8 +319,8 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
   const int len = a.lens[b];
   int blk[U];
 #pragma unroll
-  for (int u = 0; u < U; ++u) blk[u] = bt[min(block_index(t0 + rslot + R * u), a.max_blocks - 1)];
-  const int blk0 = bt[min(block_index(t0), a.max_blocks - 1)];
+  for (int u = 0; u < U; ++u) blk[u] = *entry(block_index((int)((uint32_t)t0 + rslot + R * u)));
+  const int blk0 = *entry(block_index(t0));
   Raw8<DT> qr[G];
   {
     const char* qb = reinterpret_cast<const char*>(a.q) +
@@ -349,7 +351,7 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
   __shared__ int s_share;
   if (NEW != kNone && wave == 3) {
     to_lds4(a.lens + min(lane, a.n_seqs - 1), s_new[0]);
-    to_lds4(bt + min(block_index(t0) + lane, a.max_blocks - 1), s_new[1]);
+    to_lds4(entry((int)((uint32_t)block_index(t0) + lane)), s_new[1]);
   }
   // RMSNorm + RoPE of one head row
   auto new_head = [&](const u32x4& raw, const u32x4& w, const Rope& r) {
@@ -452,7 +454,7 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void decode_paged_kernel(Decod
     if (t1 > t0) {
       const int first = block_index(t0), last = block_index(t1 - 1);
       for (int i0 = first; i0 <= last; i0 += 64) {
-        const int own = lds && i0 == first ? s_new[1][lane] : bt[min(i0 + lane, a.max_blocks - 1)];
+        const int own = lds && i0 == first ? s_new[1][lane] : *entry(i0 + lane);
         const int n = min(64, last + 1 - i0);
         for (int j = 0; j < n; ++j) {
           const int t = (i0 + j) * a.block_size + off;

@@ -568,3 +568,36 @@ def test_infinite_values_in_the_last_partition(gpu, dtype, append, splits):
     fin = ref.isfinite()
     assert torch.equal(out[~fin].double(), ref[~fin])
     _close_decode(out[fin], ref[fin], dtype, float(vc[vc.isfinite()].abs().max()))
+
+
+@pytest.mark.parametrize("bs", [256, 300])
+@pytest.mark.parametrize("append", [False, True])
+def test_tables_past_two_to_the_31_tokens(gpu, bs, append):
+    """A table whose capacity passes 2^31 tokens, in partitions large enough that
+    a partition starts past it: the block numbers loaded before the context length
+    is known stay inside the table, and the result is that of a short table."""
+    print(f"case: huge table block {bs} append={append}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(17)
+    W = (1 << 31) // bs + 9
+    kc = torch.randn((8, bs, 8, 128), generator=g, device=gpu).bfloat16()
+    vc = torch.randn((8, bs, 8, 128), generator=g, device=gpu).bfloat16()
+    q = torch.randn((2, 1, 16, 128), generator=g, device=gpu).bfloat16()
+    kw = {}
+    if append:
+        k, v = torch.randn((2, 2, 1, 8, 128), generator=g, device=gpu).bfloat16()
+        kw = dict(k=k, v=v)
+    sl = torch.tensor([290, 2 * bs + 1], dtype=torch.int32, device=gpu)
+    short = torch.tensor([[3, 1, 0, 2], [5, 4, 7, 6]], dtype=torch.int32, device=gpu)
+    huge = torch.zeros((2, W), dtype=torch.int32, device=gpu)
+    huge[:, :4] = short
+    part = 1 << 30
+    assert -(-W * bs // part) == 3 and 2 * part >= 1 << 31
+    ref = fai.flash_attn_with_kvcache(q, kc.clone(), vc.clone(), cache_seqlens=sl, block_table=short, **kw)
+    out = fai.flash_attn_with_kvcache(q, kc, vc, cache_seqlens=sl, block_table=huge,
+                                      num_splits=3 if append else 2, **kw)
+    torch.cuda.synchronize()
+    _close_decode(out, ref, torch.bfloat16, float(vc.float().abs().max()))
+    if not append:
+        out = fai.decode_paged(q[:, 0], kc, vc, huge, sl, partition_tokens=part)
+        torch.cuda.synchronize()
+        _close_decode(out, ref[:, 0], torch.bfloat16, float(vc.float().abs().max()))
