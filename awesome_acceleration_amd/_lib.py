@@ -60,6 +60,11 @@ SIGNATURES: dict[str, tuple] = {
         [_p, _i64, _p, _p, _i64, _i64, _p, _p, _i64, _i32, _p, _i32, _p, _i32, _i32, _i32, _i32,
          _i32, _f32, _p, _i64, _p, _size, _i32, _i32, _p],
     ),
+    "aac_decode_append_merge_paged": (
+        _c_int,
+        [_p, _i64, _p, _p, _i64, _i64, _p, _p, _i64, _i32, _p, _i32, _p, _i32, _i32, _i32, _i32,
+         _i32, _f32, _p, _i64, _p, _size, _p, _i32, _i32, _p],
+    ),
     "aac_decode_qkv_paged": (
         _c_int,
         [_p, _i64, _p, _p, _f32, _p, _p, _i32, _p, _p, _p, _i64, _i32, _p, _i32, _p, _i32, _i32,

@@ -965,6 +965,7 @@ extern "C" size_t aac_decode_workspace_bytes(int32_t n_seqs, int32_t n_q_heads, 
 struct NewToken {
   const void *k = nullptr, *v = nullptr;
   int64_t k_stride = 0, v_stride = 0;
+  void* counters = nullptr;  // [n_seqs, n_kv_heads] x 8 bytes, or null
   const void *qw = nullptr, *kw = nullptr, *cos = nullptr, *sin = nullptr;
   const int32_t* positions = nullptr;
   int32_t max_pos = 0;
@@ -1046,18 +1047,14 @@ static int decode_common(const void* q, int64_t q_seq_stride, const void* k_cach
   if (plan.ws_bytes) {
     a.ws_o = reinterpret_cast<float*>(workspace);
     a.ws_lse = a.ws_o + (size_t)n_seqs * n_q_heads * plan.n_parts * kHeadDim;
-    // Room for counters past the partial results: a small append call combines
-    // them in its launch.  Writes past the L2s, the counting and the second read
-    // take the GPU longer than a second launch from some 4 partitions on (24
-    // sequences in 9 partitions 29.9 us against 25.7), but a caller that launches
-    // each call itself is bound by its launches (fp32, 4 sequences in 8
-    // partitions: 15.3 us a call with the second launch, 13.5 without).  The room
-    // is the caller's choice.
-    const size_t cnt = (plan.ws_bytes + 15) / 16 * 16;
-    const int64_t items = (int64_t)n_seqs * n_kv_heads;
-    if (nt.k && !nt.qw && plan.n_parts <= 8 && items * plan.n_parts <= 512 &&
-        workspace_bytes >= cnt + (size_t)items * 8)
-      a.ws_cnt = reinterpret_cast<unsigned long long*>((char*)workspace + cnt);
+    // With counters a small append call combines its partitions in its launch.
+    // Writes past the L2s, the counting and the second read take the GPU longer than
+    // a second launch from some 4 partitions on (24 sequences in 9 partitions 29.9 us
+    // against 25.7), but a caller that launches each call itself is bound by its
+    // launches (fp32, 4 sequences in 8 partitions: 15.3 us a call with the second
+    // launch, 13.5 without).
+    if (nt.counters && plan.n_parts <= 8 && (int64_t)n_seqs * n_kv_heads * plan.n_parts <= 512)
+      a.ws_cnt = reinterpret_cast<unsigned long long*>(nt.counters);
   }
   a.k_new = nt.k;
   a.v_new = nt.v;
@@ -1146,21 +1143,19 @@ extern "C" int aac_decode_paged_noalloc(const void* q, int64_t q_seq_stride, con
   return decode_common(q, q_seq_stride, k_cache, v_cache, num_blocks, block_size, block_tables,
                        max_blocks_per_seq, context_lens, 0, n_seqs, max_context_len, n_q_heads,
                        n_kv_heads, head_dim, scale, out, out_seq_stride, ws,
-                       need, partition_tokens, dtype,
+                       need ? (size_t)AAC_DECODE_SCRATCH_BYTES : 0, partition_tokens, dtype,
                        (hipStream_t)stream);
 }
 
-extern "C" int aac_decode_append_paged(const void* q, int64_t q_seq_stride, const void* k,
-                                       const void* v, int64_t k_tok_stride, int64_t v_tok_stride,
-                                       void* k_cache, void* v_cache, int64_t num_blocks,
-                                       int32_t block_size, const int32_t* block_tables,
-                                       int32_t max_blocks_per_seq, const int32_t* cache_seqlens,
-                                       int32_t n_seqs, int32_t max_context_len, int32_t n_q_heads,
-                                       int32_t n_kv_heads, int32_t head_dim, float scale, void* out,
-                                       int64_t out_seq_stride, void* workspace,
-                                       size_t workspace_bytes, int32_t partition_tokens,
-                                       int32_t dtype, void* stream) {
+extern "C" int aac_decode_append_merge_paged(
+    const void* q, int64_t q_seq_stride, const void* k, const void* v, int64_t k_tok_stride,
+    int64_t v_tok_stride, void* k_cache, void* v_cache, int64_t num_blocks, int32_t block_size,
+    const int32_t* block_tables, int32_t max_blocks_per_seq, const int32_t* cache_seqlens,
+    int32_t n_seqs, int32_t max_context_len, int32_t n_q_heads, int32_t n_kv_heads,
+    int32_t head_dim, float scale, void* out, int64_t out_seq_stride, void* workspace,
+    size_t workspace_bytes, void* counters, int32_t partition_tokens, int32_t dtype, void* stream) {
   if (head_dim != kHeadDim) return AAC_ERR_UNSUPPORTED;
+  if ((uintptr_t)counters % 8) return AAC_ERR_MISALIGNED;
   // The append runs inside the attention launch when its rows suit the 16-byte
   // loads there and there are at most 64 of them, a lane each in the search for
   // shared blocks; anything else takes the general append first (graph replay, one
@@ -1177,6 +1172,7 @@ extern "C" int aac_decode_append_paged(const void* q, int64_t q_seq_stride, cons
     nt.v = v;
     nt.k_stride = k_tok_stride;
     nt.v_stride = v_tok_stride;
+    nt.counters = counters;
     return decode_common(q, q_seq_stride, k_cache, v_cache, num_blocks, block_size, block_tables,
                          max_blocks_per_seq, cache_seqlens, 1, n_seqs, max_context_len, n_q_heads,
                          n_kv_heads, head_dim, scale, out, out_seq_stride, workspace,
@@ -1190,6 +1186,24 @@ extern "C" int aac_decode_append_paged(const void* q, int64_t q_seq_stride, cons
                        max_blocks_per_seq, cache_seqlens, 1, n_seqs, max_context_len, n_q_heads,
                        n_kv_heads, head_dim, scale, out, out_seq_stride, workspace,
                        workspace_bytes, partition_tokens, dtype, (hipStream_t)stream);
+}
+
+extern "C" int aac_decode_append_paged(const void* q, int64_t q_seq_stride, const void* k,
+                                       const void* v, int64_t k_tok_stride, int64_t v_tok_stride,
+                                       void* k_cache, void* v_cache, int64_t num_blocks,
+                                       int32_t block_size, const int32_t* block_tables,
+                                       int32_t max_blocks_per_seq, const int32_t* cache_seqlens,
+                                       int32_t n_seqs, int32_t max_context_len, int32_t n_q_heads,
+                                       int32_t n_kv_heads, int32_t head_dim, float scale, void* out,
+                                       int64_t out_seq_stride, void* workspace,
+                                       size_t workspace_bytes, int32_t partition_tokens,
+                                       int32_t dtype, void* stream) {
+  return aac_decode_append_merge_paged(q, q_seq_stride, k, v, k_tok_stride, v_tok_stride, k_cache,
+                                       v_cache, num_blocks, block_size, block_tables,
+                                       max_blocks_per_seq, cache_seqlens, n_seqs, max_context_len,
+                                       n_q_heads, n_kv_heads, head_dim, scale, out, out_seq_stride,
+                                       workspace, workspace_bytes, nullptr, partition_tokens, dtype,
+                                       stream);
 }
 
 extern "C" int aac_decode_qkv_paged(

@@ -513,13 +513,15 @@ def flash_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, rotary_cos=None
         part = max(1, math.ceil(cap / int(num_splits)))
     L = _lib.lib()
     ws_bytes = _decode_ws_bytes(B, Hq, hkv, D, bs, mb, mcl, part)
-    wsp = None
+    wsp = counters = None
     if ws_bytes:
-        # an eager append of few sequences is bound by its launches: with room for
-        # counters one launch also combines the partitions
-        if k is not None and B * hkv <= 128 and not torch.cuda.is_current_stream_capturing():
-            ws_bytes = (ws_bytes + 15) // 16 * 16 + B * hkv * 8
-        wsp = _workspace(ws_bytes, q.device).data_ptr()
+        # an eager append of few sequences is bound by its launches: with counters one
+        # launch also combines the partitions
+        merge = k is not None and B * hkv <= 128 and not torch.cuda.is_current_stream_capturing()
+        at = (ws_bytes + 15) // 16 * 16
+        wsp = _workspace(at + B * hkv * 8 if merge else ws_bytes, q.device).data_ptr()
+        if merge:
+            counters = wsp + at
     if k is None:
         rc = L.aac_decode_paged(
             q3.data_ptr(), q_stride, k_cache.data_ptr(), v_cache.data_ptr(), nblk, bs,
@@ -542,10 +544,10 @@ def flash_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, rotary_cos=None
         v = v.reshape(B, hkv, D).contiguous()
         vst = (hkv * D,)
     ks, vs = (kst[0], vst[0]) if B > 1 else (hkv * D, hkv * D)
-    rc = L.aac_decode_append_paged(
+    rc = L.aac_decode_append_merge_paged(
         q3.data_ptr(), q_stride, k.data_ptr(), v.data_ptr(), ks, vs, k_cache.data_ptr(),
         v_cache.data_ptr(), nblk, bs, tables.data_ptr(), mb, seqlens.data_ptr(), B, mcl, Hq, hkv,
-        D, _scale(softmax_scale, D), out.data_ptr(), Hq * D, wsp, ws_bytes, part,
+        D, _scale(softmax_scale, D), out.data_ptr(), Hq * D, wsp, ws_bytes, counters, part,
         _dtype_code(q), _stream(q))
-    _lib.check(rc, "aac_decode_append_paged")
+    _lib.check(rc, "aac_decode_append_merge_paged")
     return out

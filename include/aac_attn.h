@@ -173,10 +173,7 @@ int aac_prefill_varlen_store(const void* q, const void* k, const void* v, int64_
  * Bytes of split-K workspace aac_decode_paged needs for this shape.
  * max_context_len <= 0 means "table capacity" (max_blocks_per_seq *
  * block_size), partition_tokens <= 0 means "library's choice".  Returns 0
- * when the chosen plan needs no workspace.  A workspace_bytes larger by 8 bytes
- * per (sequence, KV head) past this size rounded up to 16 lets a small append call
- * combine its partitions in the attention launch instead of a second one; the
- * workspace needs no initialisation, and a call uses no more of it than that.
+ * when the chosen plan needs no workspace.
  */
 size_t aac_decode_workspace_bytes(int32_t n_seqs, int32_t n_q_heads, int32_t n_kv_heads,
                                   int32_t head_dim, int32_t block_size, int32_t max_blocks_per_seq,
@@ -256,6 +253,22 @@ int aac_decode_append_paged(const void* q, int64_t q_seq_stride, const void* k, 
                             void* out, int64_t out_seq_stride, void* workspace,
                             size_t workspace_bytes, int32_t partition_tokens, int32_t dtype,
                             void* stream);
+
+/*
+ * aac_decode_append_paged with counters (8 bytes per (sequence, KV head), 8-byte
+ * aligned, or null): a small split call then combines its partitions in the
+ * attention launch instead of a second one.  One launch less for a caller that
+ * launches each call itself; slower on the GPU from some 4 partitions on, so a
+ * captured step passes null.  The counters need no initialisation; like the
+ * workspace they belong to one call at a time.
+ */
+int aac_decode_append_merge_paged(
+    const void* q, int64_t q_seq_stride, const void* k, const void* v, int64_t k_tok_stride,
+    int64_t v_tok_stride, void* k_cache, void* v_cache, int64_t num_blocks, int32_t block_size,
+    const int32_t* block_tables, int32_t max_blocks_per_seq, const int32_t* cache_seqlens,
+    int32_t n_seqs, int32_t max_context_len, int32_t n_q_heads, int32_t n_kv_heads,
+    int32_t head_dim, float scale, void* out, int64_t out_seq_stride, void* workspace,
+    size_t workspace_bytes, void* counters, int32_t partition_tokens, int32_t dtype, void* stream);
 
 /*
  * The same step from the rows of the fused QKV projection, qkv

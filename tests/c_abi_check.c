@@ -26,7 +26,8 @@ int main(void) {
   /* every other entry point is referenced, so a missing export fails the link */
   void* volatile refs[] = {(void*)aac_kv_append_paged, (void*)aac_prefill_varlen_store,
                            (void*)aac_prefill_workspace_bytes, (void*)aac_decode_paged,
-                           (void*)aac_decode_append_paged, (void*)aac_rmsnorm,
+                           (void*)aac_decode_append_paged, (void*)aac_decode_append_merge_paged,
+                           (void*)aac_decode_qkv_paged, (void*)aac_rmsnorm_gemm_nt, (void*)aac_rmsnorm,
                            (void*)aac_qk_norm_rope_store, (void*)aac_silu_mul, (void*)aac_gemm_nt,
                            (void*)aac_qkv_norm_rope_store, (void*)aac_argmax_rows,
                            (void*)aac_kv_export_paged, (void*)aac_kv_import_paged};

@@ -601,3 +601,109 @@ def test_tables_past_two_to_the_31_tokens(gpu, bs, append):
         out = fai.decode_paged(q[:, 0], kc, vc, huge, sl, partition_tokens=part)
         torch.cuda.synchronize()
         _close_decode(out, ref[:, 0], torch.bfloat16, float(vc.float().abs().max()))
+
+
+def _small_append(gpu, seed):
+    """Four sequences of 64-1000 tokens whose bf16 plan has eight partitions; the
+    workspace's size covers fp32's twice as many."""
+    g = torch.Generator(device=gpu).manual_seed(seed)
+    kc = torch.randn((16, 256, 8, 128), generator=g, device=gpu).bfloat16()
+    vc = torch.randn((16, 256, 8, 128), generator=g, device=gpu).bfloat16()
+    bt = torch.randperm(16, generator=g, device=gpu).view(4, 4).to(torch.int32)
+    sl = torch.tensor([64, 500, 777, 999], dtype=torch.int32, device=gpu)
+    q = torch.randn((4, 1, 16, 128), generator=g, device=gpu).bfloat16()
+    k, v = torch.randn((2, 4, 1, 8, 128), generator=g, device=gpu).bfloat16()
+    return q, k, v, kc, vc, bt, sl
+
+
+def _raw_append(q, k, v, kc, vc, bt, sl, out, ws, counters):
+    from awesome_acceleration_amd import _lib
+    L = _lib.lib()
+    size = L.aac_decode_workspace_bytes(4, 16, 8, 128, 256, 4, 0, 0)
+    head = (q.data_ptr(), 16 * 128, k.data_ptr(), v.data_ptr(), 8 * 128, 8 * 128, kc.data_ptr(),
+            vc.data_ptr(), 16, 256, bt.data_ptr(), 4, sl.data_ptr(), 4, 0, 16, 8, 128, 128 ** -0.5,
+            out.data_ptr(), 16 * 128, ws.data_ptr(), size)
+    tail = (0, _lib.AAC_DTYPE[q.dtype], torch.cuda.current_stream().cuda_stream)
+    rc = (L.aac_decode_append_paged(*head, *tail) if counters is None
+          else L.aac_decode_append_merge_paged(*head, counters.data_ptr(), *tail))
+    assert rc == 0
+
+
+def test_partitions_are_combined_in_the_launch_only_with_counters(gpu):
+    """A workspace of exactly the size asked for (the fp32 plan's, twice what bf16
+    needs) does not imply the in-launch combination: nothing past the bf16 plan's
+    partial results is written.  With counters, whatever they hold, the result is
+    the same, and they are ready for the next call."""
+    print("case: combination needs counters", flush=True)
+    from awesome_acceleration_amd import _lib
+    q, k, v, kc, vc, bt, sl = _small_append(gpu, 18)
+    ref = fai.flash_attn_with_kvcache(q, kc.clone(), vc.clone(), k=k, v=v, cache_seqlens=sl, block_table=bt)
+    size = _lib.lib().aac_decode_workspace_bytes(4, 16, 8, 128, 256, 4, 0, 0)
+    plan = 4 * 16 * 8 * 129 * 4  # sequences, heads, partitions of 128 tokens
+    assert size >= plan + 4 * 8 * 8, (size, plan)
+    vmax = float(vc.float().abs().max())
+    ws = torch.full((size,), 0x5a, dtype=torch.uint8, device=gpu)
+    out = torch.full_like(q, float("nan"))
+    _raw_append(q, k, v, kc.clone(), vc.clone(), bt, sl, out, ws, None)
+    torch.cuda.synchronize()
+    assert bool((ws[plan:] == 0x5a).all())
+    _close_decode(out, ref, torch.bfloat16, vmax)
+    for fill in (0, -1, 7):
+        counters = torch.full((32,), fill, dtype=torch.int64, device=gpu)
+        for _ in range(3):
+            out = torch.full_like(q, float("nan"))
+            _raw_append(q, k, v, kc.clone(), vc.clone(), bt, sl, out, ws, counters)
+            torch.cuda.synchronize()
+            _close_decode(out, ref, torch.bfloat16, vmax)
+            # sequence 0 has one partition and does not count
+            assert counters[8:].unique().numel() == 1 and int(counters[8]) != fill
+
+
+def test_captured_append_combines_in_a_second_launch(gpu, monkeypatch):
+    """flash_attn_with_kvcache gives counters to an eager call and none under
+    capture; and a capture of the C entry with counters replays as often as wanted,
+    eager calls between."""
+    print("case: captured append", flush=True)
+    from awesome_acceleration_amd import _lib
+    q, k, v, kc, vc, bt, sl = _small_append(gpu, 19)
+    given = []
+    real = _lib.lib()
+
+    class Spy:
+        def __getattr__(self, name):
+            f = getattr(real, name)
+            if name != "aac_decode_append_merge_paged":
+                return f
+            return lambda *a: (given.append(a[-4]), f(*a))[1]
+
+    def call():
+        return fai.flash_attn_with_kvcache(q, kc, vc, k=k, v=v, cache_seqlens=sl, block_table=bt)
+
+    monkeypatch.setattr(_lib, "lib", lambda: Spy())
+    ref = call()
+    assert given[-1] is not None
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    assert given[-1] is None
+    monkeypatch.undo()
+    size = real.aac_decode_workspace_bytes(4, 16, 8, 128, 256, 4, 0, 0)
+    ws = torch.empty(size, dtype=torch.uint8, device=gpu)
+    counters = torch.full((32,), 123, dtype=torch.int64, device=gpu)
+    raw = torch.empty_like(q)
+    torch.cuda.synchronize()
+    merged = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(merged):
+        _raw_append(q, k, v, kc, vc, bt, sl, raw, ws, counters)
+    vmax = float(vc.float().abs().max())
+    for _ in range(4):
+        out.fill_(float("nan"))
+        raw.fill_(float("nan"))
+        graph.replay()
+        merged.replay()
+        again = call()
+        torch.cuda.synchronize()
+        assert torch.equal(again, ref)
+        _close_decode(out, ref, torch.bfloat16, vmax)
+        _close_decode(raw, ref, torch.bfloat16, vmax)
