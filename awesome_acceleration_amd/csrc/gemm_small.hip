@@ -388,6 +388,11 @@ int launch_small(const Args& a, int n_out, bool silu, bool f16, hipStream_t st) 
 
 using namespace aac;
 
+// Whether [a, a + na) and [b, b + nb) share a byte (null: nothing).
+static bool overlap(const void* a, size_t na, const void* b, size_t nb) {
+  return a && b && (uintptr_t)a < (uintptr_t)b + nb && (uintptr_t)b < (uintptr_t)a + na;
+}
+
 extern "C" int aac_rmsnorm_gemm_nt(const void* x, int64_t x_row_stride, const void* residual,
                                    void* residual_out, const void* norm_weight, float eps,
                                    const void* w, int64_t w_row_stride, void* y, int64_t y_row_stride,
@@ -406,6 +411,12 @@ extern "C" int aac_rmsnorm_gemm_nt(const void* x, int64_t x_row_stride, const vo
       y_row_stride % 4)
     return AAC_ERR_MISALIGNED;
   if (cdiv(m, 8) * (n / 8) >= (int64_t(1) << 31)) return AAC_ERR_UNSUPPORTED;
+  // every workgroup reads all rows of x and residual, with no order between them
+  const size_t rows = (size_t)m * k * 2, xb = ((size_t)(m - 1) * x_row_stride + k) * 2;
+  const size_t yb = ((size_t)(m - 1) * y_row_stride + n) * 2;
+  if (overlap(residual_out, rows, x, xb) || overlap(residual_out, rows, residual, rows) ||
+      overlap(y, yb, x, xb) || overlap(y, yb, residual, rows) || overlap(y, yb, residual_out, rows))
+    return AAC_ERR_INVALID_ARGUMENT;
   gs::Args a{};
   a.x = (const u16*)x;
   a.x_stride = x_row_stride;

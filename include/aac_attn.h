@@ -386,9 +386,10 @@ int aac_qkv_norm_rope_store(const void* x, int64_t x_row_stride, const void* w_q
 /*
  * aac_gemm_nt with the residual add and RMSNorm of aac_rmsnorm in its
  * prologue, for a decode step of few rows: h = x, or h = dtype(x + residual)
- * with residual_out = h when residual is given (both contiguous [m, k]; not
- * the same buffer), y = norm(h) w^T (with silu_intermediate: SiLU * up).  k is
- * 512 or 1024 and n a multiple of 32, else AAC_ERR_UNSUPPORTED.
+ * with residual_out = h when residual is given (both contiguous [m, k]),
+ * y = norm(h) w^T (with silu_intermediate: SiLU * up).  k is 512 or 1024 and n a
+ * multiple of 32, else AAC_ERR_UNSUPPORTED.  Not in place: residual_out and y share
+ * no byte with x, residual or each other, else AAC_ERR_INVALID_ARGUMENT.
  */
 int aac_rmsnorm_gemm_nt(const void* x, int64_t x_row_stride, const void* residual,
                         void* residual_out, const void* norm_weight, float eps, const void* w,

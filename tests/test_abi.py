@@ -113,6 +113,29 @@ def test_host_side_argument_rejection():
     assert ex(16, 0, 0, 2, 4, 16, 8, 128, 64, 1, 8, 24, 0, None) == -3
 
 
+def test_norm_projection_refuses_to_run_in_place():
+    """aac_rmsnorm_gemm_nt: every workgroup reads all rows of x and the residual, so
+    an output that shares bytes with them, in whole or in part, is refused before
+    any launch."""
+    f = _lib.lib().aac_rmsnorm_gemm_nt
+    m, n, k = 4, 128, 512
+    row = 2 * k
+    x, res, out, nw, w, y = (1 << 30) + 0x100000, 0x20000000, 0x30000000, 0x40000000, 0x50000000, 0x60000000
+
+    def call(x=x, xs=k, res=res, out=out, y=y):
+        return f(x, xs, res, out, nw, 1e-6, w, k, y, n, m, n, k, 0, 0, None)
+
+    assert call(out=res) == -1
+    assert call(out=x) == -1
+    assert call(out=res + (m - 1) * row) == -1            # the last row only
+    assert call(res=out + 16 * 3) == -1
+    assert call(xs=2 * k, out=x + (m - 1) * 2 * row) == -1  # the last row of a strided x
+    assert call(y=x) == -1
+    assert call(y=res + 8) == -1
+    assert call(y=out) == -1
+    assert call(res=None, out=None, y=x + m * row - 8) == -1
+
+
 def test_workspace_sizing():
     L = _lib.lib()
     # context that fits one partition needs no workspace
