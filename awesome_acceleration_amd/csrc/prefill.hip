@@ -666,9 +666,10 @@ static int launch_g(const Args& a, int g, int max_q, int n_cu, hipStream_t st) {
 // 1 x 4096 111.9 -> 92.0; not split because it measured slower: 256 items
 // of at most 16 tiles (8 x 1024 at 8/4 heads 34.8 -> 43.0, 4 x 1024 at 16/8
 // 34.0 -> 43.3), items under 16 tiles (1 x 512 19.0 -> 19.4, 2 x 256
-// 12.3 -> 15.9); four pieces never beat two by more than noise.  Calls with groups
-// of 2, 4 and 8 that this plan would split run on prefill_split.hip instead (1 x
-// 1024 at 16/8 heads 14.5 us, 1 x 2048 29.2); it serves group 1.
+// 12.3 -> 15.9); four pieces never beat two by more than noise.  Of the calls with
+// groups of 2, 4 and 8 prefill_split.hip takes most that this plan would split (1 x
+// 1024 at 16/8 heads 14.5 us, 1 x 2048 29.2; its lines stand there); the plan serves
+// group 1 and calls with many more keys than queries.
 struct SplitPlan {
   int32_t n_split;
   int64_t n_items;  // items (without pieces): counters in the workspace
@@ -784,11 +785,13 @@ static int prefill_common(const void* q, const void* k, const void* v, int64_t q
   // that kernel's loads may reach 128 rows past a segment's keys: their (out of
   // range) offsets stay in 32 bits
   const bool reach = ((int64_t)max_seqlen_k + 160) * std::max(k_tok_stride, v_tok_stride) * 2 < (int64_t(1) << 31);
-  const int slices =
-      reach ? prefill_split_slices(g, scale, n_seqs, n_kv_heads, max_seqlen_q, max_seqlen_k, n_cu) : 0;
+  if (workspace_bytes < sp.ws_bytes) sp = {1, 0, 0};
+  const int slices = reach ? prefill_split_slices(g, scale, n_seqs, n_kv_heads, max_seqlen_q, max_seqlen_k,
+                                                  causal != 0, n_cu, sp.n_split * sp.n_items <= n_cu && sp.n_split > 1)
+                           : 0;
   if (slices) {
     rc = prefill_split_launch(a, slices, g, causal != 0, n_store > 0, f16, max_seqlen_q, stream);
-  } else if (sp.n_split > 1 && workspace_bytes >= sp.ws_bytes) {
+  } else if (sp.n_split > 1) {
     a.n_split = sp.n_split;
     a.ws_cnt = reinterpret_cast<int32_t*>(workspace);
     a.ws_o = reinterpret_cast<float*>((char*)workspace + pf::kCntBytes);
@@ -826,8 +829,15 @@ extern "C" size_t aac_prefill_workspace_bytes(int32_t n_seqs, int32_t max_seqlen
   if (head_dim != pf::D) return 0;
   int n_cu = 0;
   if (device_cu_count(&n_cu) != AAC_OK) return 0;
-  return pf::plan_split(n_seqs, max_seqlen_q, max_seqlen_k, n_q_heads, n_kv_heads, causal != 0, n_cu)
-      .ws_bytes;
+  const pf::SplitPlan sp =
+      pf::plan_split(n_seqs, max_seqlen_q, max_seqlen_k, n_q_heads, n_kv_heads, causal != 0, n_cu);
+  // none where prefill_split.hip takes the call (for a positive scale and strides
+  // well below 2 GiB; other calls then run unsplit)
+  if (sp.n_split > 1 &&
+      prefill_split_slices(n_q_heads / n_kv_heads, 1.f, n_seqs, n_kv_heads, max_seqlen_q, max_seqlen_k,
+                           causal != 0, n_cu, sp.n_split * sp.n_items <= n_cu))
+    return 0;
+  return sp.ws_bytes;
 }
 
 extern "C" int aac_prefill_varlen(const void* q, const void* k, const void* v, int64_t q_tok_stride,

@@ -341,7 +341,11 @@ static void launch_t(const Args& a, bool four, unsigned grid, hipStream_t st) {
 }  // namespace ps
 
 // Where the lines lie, by items (32 queries of two heads) per CU.  Measured on
-// MI355X (causal, graph replay, us): W the wide kernel, 4 and 2 the slices here.
+// MI355X (graph replay, us): W the wide kernel, P the eight-wave kernel's two pieces
+// per item, 4 and 2 the slices here; over 1,794 shapes of 16-2048 queries, up to
+// 32,768 keys and groups 2, 4 and 8 the choice is at most 5% behind W or P.
+//
+// Causal, with keys for the queries alone or half as many more:
 //   up to one item: 16/8 heads, 1 x 128 W 11.5, 4 6.4, 2 5.7; 1 x 256 12.9, 7.5,
 //     7.5; 1 x 777 23.3, 12.1, 15.1 (with the store 24.8, 12.9); 1 x 1024 28.6,
 //     14.5, 18.9: four slices for more than 256 keys
@@ -349,23 +353,50 @@ static void launch_t(const Args& a, bool four, unsigned grid, hipStream_t st) {
 //     3 x 1024 28.4, 17.9, 19.3: four from 640 keys on
 //   up to three: 6 x 512 W 19.0, 2 15.9; 1 x 3072 69.1, 57.0; 12 x 250 13.1, 11.8
 //   up to four: 1 x 4096 W 93.1, 2 84.7; 2 x 2048 50.7, 47.8, but 16 x 256 15.2,
-//     18.0: from 1024 keys on.  Beyond, the wide kernel, whose tiles serve four
-//     times the queries (8 x 1024 46.4, 55.9)
+//     18.0: from 1024 keys on; where there are more keys than queries from 3072 on
+//     (4 x 1024 queries, 1536 keys W 44.3, 2 50.5).  Beyond, the wide kernel, whose
+//     tiles serve four times the queries (8 x 1024 46.4, 55.9)
 //   segments of one block of 32 queries keep one of its four waves busy: 256 x 32
 //     at 16/8 heads W 50.3, 2 21.6, at 32/8 55.5, 33.4; of two blocks 57.0, 40.8,
 //     but at 32/8 67.7, 82.0
-static int pick_slices(int g, int n_seqs, int hkv, int max_q, int max_k, int n_cu) {
-  const int64_t items = (int64_t)n_seqs * hkv * (g / 2) * cdiv(max_q, 32);
-  if ((items <= n_cu && max_k > 256) || (items <= 2 * (int64_t)n_cu && max_k >= 640)) return 4;
-  if (items <= 3 * (int64_t)n_cu || (items <= 4 * (int64_t)n_cu && max_k >= 1024) || max_q <= 32 ||
-      (max_q <= 64 && g == 2))
-    return 2;
-  return 0;
+//
+// Every item sees all or most of its keys (not causal, or many more keys than
+// queries).  Each item here reads them for itself, where W reads them once for 128
+// queries, and the longer they are the more of the time that is:
+//   up to one item: 16/8 heads, 8 x 128 queries, 2048 keys P 47.2, 4 30.8, 2 44.7;
+//     1 x 512, 8192 keys 133.8, 89.6, 145.6.  But when the keys and values pass
+//     the 256 MiB last-level cache the call is bound by drawing them, and P draws
+//     with twice the CUs where it finds them idle: 16 x 32, 8192 keys P 127, 4 164;
+//     8 x 64, 16,384 keys 200, 273
+//   up to two: 16 x 128, 512 keys W 21.8, 2 18.6; 64 x 32, 512 keys 34.9, 26.8; 16 x
+//     128, 2048 keys P 57.6, 2 50.7, but 32/8 32 x 32, 2048 keys W 55.7, 2 63.8
+//   up to three: 24 x 128, 160 keys W 13.8, 2 13.4; 24 x 64, 1024 keys 39, 42.  From
+//     3072 keys on P has more pieces than CUs: 12 x 256, 4096 keys P 160, 2 119
+//   beyond: 64 x 64, 4096 keys W 234, 2 409; 32 x 128, 2048 keys 72, 159; one block of
+//     queries, 256 x 32, 512 keys 134, 125, at 32/8 144, 156; 64 x 16, 256 keys at
+//     32/8 26.5, 21.6
+static int pick_slices(int g, int n_seqs, int hkv, int max_q, int max_k, bool causal, int n_cu, bool idle_pieces) {
+  const int64_t cu = n_cu, items = (int64_t)n_seqs * hkv * (g / 2) * cdiv(max_q, 32);
+  if (causal && 2 * (int64_t)max_k <= 3 * (int64_t)max_q) {
+    if ((items <= cu && max_k > 256) || (items <= 2 * cu && max_k >= 640)) return 4;
+    if (items <= 3 * cu || (items <= 4 * cu && max_k >= (max_k <= max_q ? 1024 : 3072))) return 2;
+    if (max_k <= max_q) return max_q <= 32 || (max_q <= 64 && g == 2) ? 2 : 0;
+  } else if (items <= cu) {
+    if (max_k <= 256) return 2;
+    return idle_pieces && (int64_t)n_seqs * hkv * max_k * (2 * pf::D * 2) > (int64_t(256) << 20) ? 0 : 4;
+  } else if (items <= 2 * cu) {
+    return max_k <= 1024 || (max_k <= 2048 && max_q > 32) ? 2 : 0;
+  } else if (items <= 3 * cu) {
+    return max_k <= 512 || max_k >= 3072 ? 2 : 0;
+  }
+  if (max_q <= 32) return max_k <= (g == 2 ? 512 : g == 4 ? 256 : max_q <= 16 || items <= 8 * cu ? 64 : 0) ? 2 : 0;
+  return g == 2 && max_q <= 64 && max_k <= 128 ? 2 : 0;
 }
 
-int prefill_split_slices(int g, float scale, int n_seqs, int hkv, int max_q, int max_k, int n_cu) {
+int prefill_split_slices(int g, float scale, int n_seqs, int hkv, int max_q, int max_k, bool causal, int n_cu,
+                         bool idle_pieces) {
   if ((g != 2 && g != 4 && g != 8) || !(scale > 0.f)) return 0;
-  return pick_slices(g, n_seqs, hkv, max_q, max_k, n_cu);
+  return pick_slices(g, n_seqs, hkv, max_q, max_k, causal, n_cu, idle_pieces);
 }
 
 int prefill_split_launch(const pf::Args& a0, int slices, int g, bool causal, bool store, bool f16, int max_q,

@@ -123,9 +123,11 @@ int aac_kv_append_paged(const void* k, const void* v, int64_t k_tok_stride, int6
  * numbered from its end), and only its first max_seqlen_k keys are
  * attended; no access leaves the segment's rows.  Built for dtype
  * BF16/FP16, head_dim 128, group 1/2/4/8.  With too few work items for the
- * GPU -- one or a few long requests -- the key range of each item is split
- * over two workgroups whose partial results are merged by a log-sum-exp
- * combine (in a fixed order: results are the same on every run).  The split needs `workspace` of
+ * GPU -- one or a few long requests -- the keys of each item are split over its
+ * workgroup's waves (groups 2, 4 and 8) or over two workgroups whose partial
+ * results are merged by a log-sum-exp combine (in a fixed order: results are the
+ * same on every run).  The latter, group 1's and that of groups with many more
+ * keys than queries, needs `workspace` of
  * aac_prefill_workspace_bytes(...) bytes, 256-byte aligned, ZERO-FILLED
  * ONCE when it is allocated: its first 16 KiB are per-item counters that
  * every call leaves at zero again, the rest partial results (do not share
@@ -143,7 +145,7 @@ int aac_prefill_varlen(const void* q, const void* k, const void* v, int64_t q_to
 
 /*
  * Workspace bytes aac_prefill_varlen would use to split this shape's key
- * ranges on the current device (0: the plan does not split).
+ * ranges over two workgroups on the current device (0: it would not).
  */
 size_t aac_prefill_workspace_bytes(int32_t n_seqs, int32_t max_seqlen_q, int32_t max_seqlen_k,
                                    int32_t n_q_heads, int32_t n_kv_heads, int32_t head_dim,

@@ -274,15 +274,33 @@ def _unsplit(q, k, v, cq, ck, Lq, Lk, causal, scale):
     return out
 
 
-@pytest.mark.parametrize("lens_q,lens_k,hq,hkv,causal,dtype", [
-    ([1024], [1024], 16, 8, True, torch.bfloat16),        # one request: 64 items for 256 CUs
-    ([2048] * 2, [2048] * 2, 8, 4, True, torch.bfloat16),  # a TP=2 rank's heads, 2 requests
-    ([300, 1000], [300, 1000], 16, 8, True, torch.bfloat16),
-    ([512], [2048], 32, 8, False, torch.bfloat16),          # non-causal, Lq != Lk
+# Calls whose items run in two pieces each (a workspace is asked for): one query
+# head per KV head, and groups with many more keys than queries.
+SPLIT_CALLS = [
+    ([1024], [1024], 8, 8, True, torch.bfloat16),          # one request: 32 items for 256 CUs
+    ([2048] * 2, [2048] * 2, 4, 4, True, torch.bfloat16),
+    ([300, 1000], [300, 1000], 16, 16, True, torch.bfloat16),
+    ([512], [2048], 8, 8, False, torch.float16),           # non-causal, Lq != Lk
+    ([512], [2048], 8, 8, False, torch.bfloat16),
     ([1500], [1500], 8, 8, True, torch.float16),
-    ([200, 5, 600], [260, 5, 1200], 16, 4, True, torch.bfloat16),  # Lq < Lk, bottom-right
-    ([4096], [4096], 8, 1, True, torch.bfloat16),          # group 8: one 32-query slot, 8 heads
-])
+    ([200, 5, 600], [260, 5, 1200], 8, 8, True, torch.bfloat16),  # Lq < Lk, bottom-right
+    ([224, 224, 7, 224, 223], [2100, 2099, 2100, 300, 2100], 16, 8, True, torch.bfloat16),
+    ([64] * 9, [2100] * 8 + [1], 32, 8, False, torch.bfloat16),
+    ([64] * 33, [2100] * 33, 8, 1, True, torch.float16),   # group 8: one 32-query slot, 8 heads
+]
+
+
+def _oracle_check(out, q, k, v, cq, ck, causal, what):
+    cq_np, ck_np = cq.cpu().numpy(), ck.cpu().numpy()
+    scale = 128 ** -0.5
+    ref = oracle.varlen_attention(f64(q), f64(k), f64(v), cq_np, ck_np, scale=scale, causal=causal)
+    absv = oracle.varlen_attention(f64(q), f64(k), np.abs(f64(v)), cq_np, ck_np, scale=scale,
+                                   causal=causal)
+    for name, o in out.items():
+        check_attention(o, ref, what=f"{what}: {name}", absv=absv)
+
+
+@pytest.mark.parametrize("lens_q,lens_k,hq,hkv,causal,dtype", SPLIT_CALLS)
 def test_split_keys_match_unsplit_and_oracle(gpu, lens_q, lens_k, hq, hkv, causal, dtype):
     """Few work items: the key range of every item is split over several
     workgroups and merged (log-sum-exp) by the last piece to finish.  The
@@ -294,21 +312,79 @@ def test_split_keys_match_unsplit_and_oracle(gpu, lens_q, lens_k, hq, hkv, causa
     from awesome_acceleration_amd import _lib
     q, k, v, cq, ck = _ragged(lens_q, lens_k, hq, hkv, dtype, gpu, seed=31)
     Lq, Lk = max(lens_q), max(lens_k)
-    ws = _lib.lib().aac_prefill_workspace_bytes(len(lens_q), Lq, Lk, hq, hkv, 128, int(causal))
+    L = _lib.lib()
+    ws = L.aac_prefill_workspace_bytes(len(lens_q), Lq, Lk, hq, hkv, 128, int(causal))
     assert ws > 0, "the plan should split this shape"
     scale = 128 ** -0.5
     outs = [fai.flash_attn_varlen_func(q, k, v, cq, ck, Lq, Lk, causal=causal) for _ in range(3)]
     base = _unsplit(q, k, v, cq, ck, Lq, Lk, causal, scale)
+    # the pieces did run: partial results past the counters, which are zero again
+    counters = fai._PF_COUNTER_BYTES
+    buf = torch.zeros(ws, dtype=torch.uint8, device=gpu)
+    buf[counters:] = 0x5a
+    own = torch.empty_like(q)
+    rc = L.aac_prefill_varlen(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), q.stride(0), k.stride(0), v.stride(0),
+        cq.data_ptr(), ck.data_ptr(), len(lens_q), Lq, Lk, hq, hkv, 128, scale, int(causal),
+        own.data_ptr(), own.stride(0), buf.data_ptr(), ws, _lib.AAC_DTYPE[dtype],
+        torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, L.aac_strerror(rc)
     torch.cuda.synchronize()
-    for o in outs[1:]:
+    assert not bool(buf[:counters].any()) and bool((buf[counters:] != 0x5a).any())
+    for o in outs[1:] + [own]:
         assert torch.equal(o.view(torch.int16), outs[0].view(torch.int16))
-    cq_np, ck_np = cq.cpu().numpy(), ck.cpu().numpy()
-    ref = oracle.varlen_attention(f64(q), f64(k), f64(v), cq_np, ck_np, scale=scale, causal=causal)
-    absv = oracle.varlen_attention(f64(q), f64(k), np.abs(f64(v)), cq_np, ck_np, scale=scale,
-                                   causal=causal)
-    check_attention(outs[0], ref, what="split", absv=absv)
-    check_attention(base, ref, what="unsplit", absv=absv)
+    _oracle_check({"split": outs[0], "unsplit": base}, q, k, v, cq, ck, causal, "pieces")
     assert float((outs[0].float() - base.float()).abs().max()) <= 2 ** -6
+
+
+@pytest.mark.parametrize("lens_q,lens_k,hq,hkv,causal,dtype", [
+    ([1024], [1024], 16, 8, True, torch.bfloat16),         # one request: 256 items
+    ([2048] * 2, [2048] * 2, 8, 4, True, torch.bfloat16),  # a TP=2 rank's heads, 2 requests
+    ([300, 1000], [300, 1000], 16, 8, True, torch.bfloat16),
+    ([512], [2048], 32, 8, False, torch.bfloat16),          # non-causal, Lq != Lk
+    ([200, 5, 600], [260, 5, 1200], 16, 4, True, torch.bfloat16),  # Lq < Lk, bottom-right
+    ([4096], [4096], 8, 1, True, torch.bfloat16),          # group 8
+    ([64] * 8, [4096] * 8, 16, 8, True, torch.float16),     # many more keys than queries
+    ([33, 32, 1], [3000, 256, 1], 64, 8, False, torch.bfloat16),
+])
+def test_few_items_need_no_workspace(gpu, lens_q, lens_k, hq, hkv, causal, dtype):
+    """Calls of few items with two query heads or more per KV head: the keys are
+    split over a workgroup's waves, no workspace is asked for, one that is given
+    is left alone, and the result meets the oracle's bound."""
+    print(f"case: few items q={lens_q} k={lens_k} {hq}/{hkv} causal={causal} {dtype}", flush=True)
+    from awesome_acceleration_amd import _lib
+    q, k, v, cq, ck = _ragged(lens_q, lens_k, hq, hkv, dtype, gpu, seed=32)
+    Lq, Lk = max(lens_q), max(lens_k)
+    assert _lib.lib().aac_prefill_workspace_bytes(len(lens_q), Lq, Lk, hq, hkv, 128, int(causal)) == 0
+    before = {key: t.data_ptr() for key, t in fai._pf_ws.items()}
+    out = fai.flash_attn_varlen_func(q, k, v, cq, ck, Lq, Lk, causal=causal)
+    again = _unsplit(q, k, v, cq, ck, Lq, Lk, causal, 128 ** -0.5)
+    torch.cuda.synchronize()
+    assert {key: t.data_ptr() for key, t in fai._pf_ws.items()} == before
+    assert torch.equal(out.view(torch.int16), again.view(torch.int16))
+    _oracle_check({"out": out}, q, k, v, cq, ck, causal, "few items")
+
+
+def test_keys_past_the_last_level_cache(gpu):
+    """Few queries over more keys than the last-level cache holds: two pieces per
+    item with a workspace, the keys split over a workgroup's waves without."""
+    print("case: keys past the last-level cache", flush=True)
+    from awesome_acceleration_amd import _lib
+    n, lq, lk, hq, hkv = 16, 32, 4224, 16, 8
+    g = torch.Generator(device=gpu).manual_seed(33)
+    q = torch.randn((n * lq, hq, 128), generator=g, device=gpu).bfloat16()
+    k = torch.randn((n * lk, hkv, 128), generator=g, device=gpu).bfloat16()
+    v = torch.randn((n * lk, hkv, 128), generator=g, device=gpu).bfloat16()
+    cq = torch.arange(0, n * lq + 1, lq, dtype=torch.int32, device=gpu)
+    ck = torch.arange(0, n * lk + 1, lk, dtype=torch.int32, device=gpu)
+    assert 2 * k.numel() * 2 > 256 << 20
+    assert _lib.lib().aac_prefill_workspace_bytes(n, lq, lk, hq, hkv, 128, 1) > 0
+    assert _lib.lib().aac_prefill_workspace_bytes(n // 2, lq, lk, hq, hkv, 128, 1) == 0
+    out = fai.flash_attn_varlen_func(q, k, v, cq, ck, lq, lk, causal=True)
+    base = _unsplit(q, k, v, cq, ck, lq, lk, True, 128 ** -0.5)
+    torch.cuda.synchronize()
+    assert not torch.equal(out, base)
+    assert float((out.float() - base.float()).abs().max()) <= 2 ** -6
 
 
 def test_split_workspace_reused_by_a_call_with_more_items(gpu):
@@ -318,10 +394,10 @@ def test_split_workspace_reused_by_a_call_with_more_items(gpu):
     ever overwrites, so every row of the later call is written."""
     print("case: split workspace reuse, few then many items", flush=True)
     from awesome_acceleration_amd import _lib
-    small = _ragged([1024], [1024], 16, 8, torch.bfloat16, gpu, seed=41)      # 64 items, split
-    big = _ragged([2048] * 2, [2048] * 2, 8, 4, torch.bfloat16, gpu, seed=42)  # 128 items, split
-    assert _lib.lib().aac_prefill_workspace_bytes(1, 1024, 1024, 16, 8, 128, 1) > 0
-    assert _lib.lib().aac_prefill_workspace_bytes(2, 2048, 2048, 8, 4, 128, 1) > 0
+    small = _ragged([1024], [1024], 8, 8, torch.bfloat16, gpu, seed=41)        # 32 items, split
+    big = _ragged([2048] * 2, [2048] * 2, 8, 8, torch.bfloat16, gpu, seed=42)  # 128 items, split
+    assert _lib.lib().aac_prefill_workspace_bytes(1, 1024, 1024, 8, 8, 128, 1) > 0
+    assert _lib.lib().aac_prefill_workspace_bytes(2, 2048, 2048, 8, 8, 128, 1) > 0
     for (q, k, v, cq, ck) in (small, big, small, big):
         L = int((cq[1:] - cq[:-1]).max())
         out = torch.full_like(q, float("nan"))
@@ -329,6 +405,7 @@ def test_split_workspace_reused_by_a_call_with_more_items(gpu):
         base = _unsplit(q, k, v, cq, ck, L, L, True, 128 ** -0.5)
         torch.cuda.synchronize()
         assert torch.isfinite(out.float()).all()
+        assert not torch.equal(out, base)  # another order of the same sums
         assert float((out.float() - base.float()).abs().max()) <= 2 ** -6
 
 
@@ -336,7 +413,8 @@ def test_split_workspace_reused_by_a_call_with_more_items(gpu):
     (16, 8, torch.bfloat16, True, [1024] * 8),             # the 8 x 1024 layer
     (32, 8, torch.bfloat16, True, [3000, 17, 700]),         # GQA-4, ragged
     (16, 8, torch.float16, False, [300, 1500]),            # fp16, non-causal
-    (16, 8, torch.bfloat16, True, [2048]),                  # one request: split key ranges
+    (16, 8, torch.bfloat16, True, [2048]),                  # one request: keys split over waves
+    (8, 8, torch.bfloat16, True, [2048]),                   # one request: items in two pieces
 ])
 def test_constant_values_return_that_value(gpu, hq, hkv, dtype, causal, lens):
     """Every V row of KV head h equal to one vector u_h: every query row returns
@@ -372,10 +450,10 @@ def test_split_prefills_on_two_streams_keep_their_own_workspaces(gpu):
     results), so each result equals the same call made alone, bit for bit."""
     print("case: split prefills on two streams", flush=True)
     from awesome_acceleration_amd import _lib
-    a = _ragged([2048], [2048], 16, 8, torch.bfloat16, gpu, seed=51)
-    b = _ragged([1536], [1536], 16, 8, torch.bfloat16, gpu, seed=52)
-    assert _lib.lib().aac_prefill_workspace_bytes(1, 2048, 2048, 16, 8, 128, 1) > 0
-    assert _lib.lib().aac_prefill_workspace_bytes(1, 1536, 1536, 16, 8, 128, 1) > 0
+    a = _ragged([2048], [2048], 16, 16, torch.bfloat16, gpu, seed=51)
+    b = _ragged([1536], [1536], 16, 16, torch.bfloat16, gpu, seed=52)
+    assert _lib.lib().aac_prefill_workspace_bytes(1, 2048, 2048, 16, 16, 128, 1) > 0
+    assert _lib.lib().aac_prefill_workspace_bytes(1, 1536, 1536, 16, 16, 128, 1) > 0
 
     def call(x):
         q, k, v, cq, ck = x
