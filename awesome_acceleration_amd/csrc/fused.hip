@@ -119,7 +119,9 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(QkArgs a) {
 // Many tokens (a prefill chunk): one wavefront per token; its four DPP rows
 // take the heads in turn (row r: heads r, r + 4, ...), so the token's
 // position, cos/sin vectors, norm weights and cache row are fetched once,
-// and a row loads a group of its heads before it processes the first.
+// and a row loads a group of its heads before it processes the first.  (fp16 takes
+// 82 registers; held to 80 by three heads a group or a launch bound 16,000 tokens
+// take 51.5 us against 50.3, 24,000 88 against 85.)
 template <Dt DT, bool NT>
 __global__ __launch_bounds__(256) void qk_norm_rope_tok_kernel(QkArgs a) {
   const int lane = threadIdx.x & 63;

@@ -329,10 +329,13 @@ static void launch_t(Args a, int n_out, hipStream_t st) {
   a.n_tiles = n_out / WR;
   const dim3 grid((unsigned)(cdiv(a.m, XR) * a.n_tiles)), block(64 * KS);
   // k up to 1024 has two units per wave: less LDS, more workgroups per CU
-  if (NORMK == 0 && a.k > 2 * KS * kUnitK)
-    hipLaunchKernelGGL((small_kernel<WR, XR, SILU, F16, NORMK, RESID, 6>), grid, block, 0, st, a);
-  else
-    hipLaunchKernelGGL((small_kernel<WR, XR, SILU, F16, NORMK, RESID, 2>), grid, block, 0, st, a);
+  if constexpr (NORMK == 0) {
+    if (a.k > 2 * KS * kUnitK) {
+      hipLaunchKernelGGL((small_kernel<WR, XR, SILU, F16, NORMK, RESID, 6>), grid, block, 0, st, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((small_kernel<WR, XR, SILU, F16, NORMK, RESID, 2>), grid, block, 0, st, a);
 }
 
 template <int WR, bool SILU, bool F16, int NORMK, bool RESID>
