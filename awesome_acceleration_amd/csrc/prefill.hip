@@ -786,7 +786,7 @@ static int prefill_common(const void* q, const void* k, const void* v, int64_t q
   // range) offsets stay in 32 bits
   const bool reach = ((int64_t)max_seqlen_k + 160) * std::max(k_tok_stride, v_tok_stride) * 2 < (int64_t(1) << 31);
   if (workspace_bytes < sp.ws_bytes) sp = {1, 0, 0};
-  const int slices = reach ? prefill_split_slices(g, scale, n_seqs, n_kv_heads, max_seqlen_q, max_seqlen_k,
+  const int slices = reach ? prefill_split_slices(g, scale, f16, n_seqs, n_kv_heads, max_seqlen_q, max_seqlen_k,
                                                   causal != 0, n_cu, sp.n_split * sp.n_items <= n_cu && sp.n_split > 1)
                            : 0;
   if (slices) {
@@ -800,7 +800,7 @@ static int prefill_common(const void* q, const void* k, const void* v, int64_t q
                        : pf::launch_g<true, false, false, true>(a, g, max_seqlen_q, n_cu, stream))
                 : (f16 ? pf::launch_g<false, true, false, true>(a, g, max_seqlen_q, n_cu, stream)
                        : pf::launch_g<false, false, false, true>(a, g, max_seqlen_q, n_cu, stream));
-  } else if (prefill_wide_supports(g, scale) &&
+  } else if (prefill_wide_takes(g, scale, f16, n_store > 0, n_seqs, n_kv_heads, max_seqlen_q, n_cu) &&
              (n_store == 0 || num_cache_rows * n_kv_heads * head_dim * 2 < (int64_t(1) << 32)))
     // the wide kernel's cache store addresses a head's rows with 32-bit offsets
     rc = prefill_wide_launch(a, g, causal != 0, n_store > 0, f16, max_seqlen_q, n_cu, stream);
@@ -831,13 +831,15 @@ extern "C" size_t aac_prefill_workspace_bytes(int32_t n_seqs, int32_t max_seqlen
   if (device_cu_count(&n_cu) != AAC_OK) return 0;
   const pf::SplitPlan sp =
       pf::plan_split(n_seqs, max_seqlen_q, max_seqlen_k, n_q_heads, n_kv_heads, causal != 0, n_cu);
-  // none where prefill_split.hip takes the call (for a positive scale and strides
-  // well below 2 GiB; other calls then run unsplit)
-  if (sp.n_split > 1 &&
-      prefill_split_slices(n_q_heads / n_kv_heads, 1.f, n_seqs, n_kv_heads, max_seqlen_q, max_seqlen_k,
-                           causal != 0, n_cu, sp.n_split * sp.n_items <= n_cu))
-    return 0;
-  return sp.ws_bytes;
+  if (sp.n_split == 1) return 0;
+  // none where prefill_split.hip takes the call, in bf16 and fp16 (for a positive
+  // scale and strides well below 2 GiB; other calls then run unsplit)
+  const bool idle = sp.n_split * sp.n_items <= n_cu;
+  for (bool f16 : {false, true})
+    if (!prefill_split_slices(n_q_heads / n_kv_heads, 1.f, f16, n_seqs, n_kv_heads, max_seqlen_q,
+                              max_seqlen_k, causal != 0, n_cu, idle))
+      return sp.ws_bytes;
+  return 0;
 }
 
 extern "C" int aac_prefill_varlen(const void* q, const void* k, const void* v, int64_t q_tok_stride,

@@ -10,8 +10,8 @@ namespace aac {
 // is the faster one (see prefill_split.hip for where the lines lie).  idle_pieces:
 // the other one is the eight-wave kernel with two pieces per item, all on CUs of
 // their own.
-int prefill_split_slices(int g, float scale, int n_seqs, int hkv, int max_q, int max_k, bool causal, int n_cu,
-                         bool idle_pieces);
+int prefill_split_slices(int g, float scale, bool f16, int n_seqs, int hkv, int max_q, int max_k, bool causal,
+                         int n_cu, bool idle_pieces);
 
 // a.n_qblocks is set by the launcher.  store: also write the K/V rows to the
 // KV cache through a.slots (causal self-attention only).

@@ -393,10 +393,22 @@ static int pick_slices(int g, int n_seqs, int hkv, int max_q, int max_k, bool ca
   return g == 2 && max_q <= 64 && max_k <= 128 ? 2 : 0;
 }
 
-int prefill_split_slices(int g, float scale, int n_seqs, int hkv, int max_q, int max_k, bool causal, int n_cu,
-                         bool idle_pieces) {
+int prefill_split_slices(int g, float scale, bool f16, int n_seqs, int hkv, int max_q, int max_k, bool causal,
+                         int n_cu, bool idle_pieces) {
   if ((g != 2 && g != 4 && g != 8) || !(scale > 0.f)) return 0;
-  return pick_slices(g, n_seqs, hkv, max_q, max_k, causal, n_cu, idle_pieces);
+  const int slices = pick_slices(g, n_seqs, hkv, max_q, max_k, causal, n_cu, idle_pieces);
+  // fp16 calls of more items would run on the eight-wave kernel (see
+  // prefill_wide_takes), which loses less on short items than the wide one: two
+  // slices only where they beat it as well (eight-wave / two: 64 x 64 queries at 16/8
+  // heads 12.9 / 16.4, 24 x 128, not causal 11.7 / 13.0, 64 x 32, 40 keys at 32/8 12.9
+  // / 16.9; 256 x 32 at 16/8 32 / 21, 6 x 512 21.5 / 21.4, 3 x 1129 36 / 27)
+  const int64_t cu = n_cu, items = (int64_t)n_seqs * hkv * (g / 2) * cdiv(max_q, 32);
+  if (!f16 || slices != 2 || 2 * items <= 3 * cu) return slices;
+  const bool keep = g == 2 && max_q <= 32 ? true
+                    : items <= 2 * cu     ? max_q > 64
+                    : items <= 3 * cu     ? max_k > 256
+                                          : items <= 4 * cu && max_k >= 1024;
+  return keep ? 2 : 0;
 }
 
 int prefill_split_launch(const pf::Args& a0, int slices, int g, bool causal, bool store, bool f16, int max_q,

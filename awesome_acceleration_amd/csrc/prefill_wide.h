@@ -6,8 +6,9 @@
 
 namespace aac {
 
-// Shapes the wide kernel serves: GQA groups 2, 4, 8, a positive scale.
-bool prefill_wide_supports(int g, float scale);
+// Whether the wide kernel takes a call: GQA groups 2, 4, 8 and a positive scale, in
+// fp16 only where it is the faster one.
+bool prefill_wide_takes(int g, float scale, bool f16, bool store, int n_seqs, int hkv, int max_q, int n_cu);
 
 // Launch on the persistent grid (min(items, n_cu) workgroups).  a.n_qblocks
 // is set by the launcher.  store: also write the K/V rows to the KV cache

@@ -51,7 +51,8 @@
 // The item body is a template of the element type: fp16 has the same MFMA
 // shapes and cycles and its own round-to-nearest-even pack.  Six fp16 requests of
 // 131-3001 tokens at 32/8 heads: 118 us against 144 with the eight-wave kernel of
-// prefill.hip (the error against 64 bits 2.5e-4 in both).
+// prefill.hip (the error against 64 bits 2.5e-4 in both); where it takes fp16 calls
+// see prefill_wide_takes.
 //
 // FLOPs per launch (the MFMA roofline): 4 * Hq * D * (visible query/key pairs).
 
@@ -482,8 +483,22 @@ static int launch_g(const Args& a, int g, int max_q, int n_cu, hipStream_t st) {
 
 }  // namespace pw
 
-bool prefill_wide_supports(int g, float scale) {
-  return (g == 2 || g == 4 || g == 8) && scale > 0.f;
+// fp16 has the eight-wave kernel of prefill.hip beside this one: shorter per item
+// (start and epilogue), slower per key tile.  Measured on 260 ragged and even fp16
+// calls of self-attention (us, eight-wave / this one): short segments 142 x 15-79 at
+// 32/8 heads 36 / 58, 65 x 49 18.6 / 26.4; with a few items per CU the last round of
+// long items decides, either way: 10 x 365-891 at 16/8 31 / 47, 3 x 1129 the other
+// way 36 / 32.  From 20 items per CU and 512 queries on this one is never behind
+// (236 x 665-876 at 16/8 1028 / 862), nor with groups of 4 from 2400 queries on
+// (6 x 131-3001 at 32/8 137 / 114; at most 4% behind), while 2 x 7904 at 8/4 take
+// 245 / 338; with the store groups of 4 are behind at any length (12 x 3436-4013
+// 1596 / 1994).  Group 8 was not measured.  bf16 has this kernel alone.
+bool prefill_wide_takes(int g, float scale, bool f16, bool store, int n_seqs, int hkv, int max_q, int n_cu) {
+  if ((g != 2 && g != 4 && g != 8) || !(scale > 0.f)) return false;
+  if (!f16) return true;
+  const int64_t items = (int64_t)n_seqs * hkv * cdiv(max_q, 256 / g);
+  if (g == 8 || (g == 4 && store)) return false;
+  return (items >= 20 * (int64_t)n_cu && max_q >= 512) || (g == 4 && max_q >= 2400);
 }
 
 int prefill_wide_launch(const pf::Args& a, int g, bool causal, bool store, bool f16, int max_q,
