@@ -874,22 +874,26 @@ static DecodePlan plan_decode(int32_t n_seqs, int32_t hq, int32_t hkv, int32_t b
     // reduction and is the fastest (64 x 1-2k at 8 KV heads 66.7 against 68.3-73
     // in partitions of 128-1024; 64 x 10-200 10.8 against 13.9-16.3), and up to
     // two iterations of tokens for any number (1 x 93: 4.9 against 6.2).  Else the
-    // smallest partition, from one iteration up, that keeps the tables' capacity
-    // within seven workgroups per CU (4 x 64-1000: 128 8.8, 192 10.4, 256 10.6,
-    // 512 13.7; 24 x 100-2063: 256 24.1, 192 26.8, 512 27.8) and the reduction at
-    // some 48 partitions (one of 30,000: 1024 25.1, 512 26.7, 128 32.9; 2 x 6-7k
-    // GQA-4: 256 18.4, 128 20.2), twice that in fp32, whose rows are twice as
-    // long (one of 20,000: 128 39.4, 256 40.7, 512 47.2).  At most 3072 (64 x
-    // 16k-32k GQA-4 over four context draws: 75.4% of HBM peak against 73.8% for
-    // 2048, 75.1% for 2560, 74.3% for 3584 and 72.5% for 4096).
+    // smallest partition, from one iteration up in whole iterations (parts of one
+    // cost a whole one: 24 x 100-2063 in 128 24.6, 192 26.8, 256 24.1), that keeps
+    // the tables' capacity within twelve workgroups per CU, sixteen in fp32 (about half
+    // of them have tokens: 46 x 49-4548 GQA-4 in 384 92, 768 93, 2048 107; 93 x 77-2504
+    // at 4 KV heads in 384 47.7, 1024 54.9; fp32, 40 x 577-1837 in 192 84, 512 105)
+    // and the reduction at some 50 partitions (one of 30,000: 1024 25.1, 512 26.7,
+    // 128 32.9; one of 25,000 at 4 KV heads: 512 17.5, 1024 23.6; 2 x 6-7k GQA-4: 256
+    // 18.4, 128 20.2), twice that in fp32, whose rows are twice as long (one of
+    // 20,000: 128 39.4, 256 40.7, 512 47.2).  At most 3072 (64 x 16k-32k GQA-4 over
+    // four context draws: 75.4% of HBM peak against 73.8% for 2048, 75.1% for 2560,
+    // 74.3% for 3584 and 72.5% for 4096).
     const int64_t items = (int64_t)n_seqs * hkv;
-    const int64_t most_parts = elem_bytes == 4 ? 96 : 48;
+    const int64_t most_parts = elem_bytes == 4 ? 96 : 52, most_groups = elem_bytes == 4 ? 4096 : 3072;
     if ((items >= 512 && cap <= 4096) || cap <= 2 * iter_tokens) {
       part = cap;
     } else {
-      part = iter_tokens;
-      while (part < 3072 && (items * cdiv(cap, part) > 1792 || cdiv(cap, part) > most_parts)) part *= 2;
-      if (part > 3072) part = 3072;
+      for (int k : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48}) {
+        part = std::min(k * iter_tokens, 3072);
+        if (items * cdiv(cap, part) <= most_groups && cdiv(cap, part) <= most_parts) break;
+      }
     }
   }
   if (part > cap) part = cap;
