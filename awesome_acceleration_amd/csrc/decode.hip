@@ -1161,16 +1161,20 @@ extern "C" int aac_decode_append_merge_paged(
   if (head_dim != kHeadDim) return AAC_ERR_UNSUPPORTED;
   if ((uintptr_t)counters % 8) return AAC_ERR_MISALIGNED;
   // The append runs inside the attention launch when its rows suit the 16-byte
-  // loads there and there are at most 64 of them, a lane each in the search for
-  // shared blocks; anything else takes the general append first (graph replay, one
-  // launch against two, us: 24 x 100-2063 25.6 and 27.1, 64 x 10-500 16.0 and 17.4,
-  // 1 x 20,000 at 32/8 heads 24.7 and 25.9; 256 x 1-2k 249.5 and 245.3).
+  // loads there, there are at most 64 of them, a lane each in the search for shared
+  // blocks, and a partition has at most 64 blocks to search; anything else takes the
+  // general append first (graph replay, one launch against two, us: 24 x 100-2063
+  // 25.6 and 27.1, 64 x 10-500 16.0 and 17.4, 1 x 20,000 at 32/8 heads 24.7 and 25.9;
+  // 256 x 1-2k 249.5 and 245.3; partitions of 192 blocks of 16, 37 x 15k 390 and 383).
   const int es = dtype == AAC_DTYPE_FP32 ? 4 : 2;
   const int g = n_kv_heads > 0 && n_q_heads > 0 && n_q_heads % n_kv_heads == 0 ? n_q_heads / n_kv_heads : 0;
   if (n_seqs > 0 && n_seqs <= 64 && (g == 1 || g == 2 || g == 4 || g == 8) && k && v && k_cache && v_cache &&
       block_tables && cache_seqlens && num_blocks > 0 && k_tok_stride >= (int64_t)n_kv_heads * head_dim &&
       v_tok_stride >= (int64_t)n_kv_heads * head_dim && ((uintptr_t)k | (uintptr_t)v) % 16 == 0 &&
-      (k_tok_stride * es) % 16 == 0 && (v_tok_stride * es) % 16 == 0) {
+      (k_tok_stride * es) % 16 == 0 && (v_tok_stride * es) % 16 == 0 && block_size > 0 &&
+      max_blocks_per_seq > 0 &&
+      plan_decode(n_seqs, n_q_heads, n_kv_heads, block_size, max_blocks_per_seq, max_context_len,
+                  partition_tokens, es).part_tokens <= 64 * (int64_t)block_size) {
     NewToken nt;
     nt.k = k;
     nt.v = v;
