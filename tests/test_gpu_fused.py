@@ -205,3 +205,53 @@ def test_argmax_matches_torch(gpu, dtype, rows, cols, pad):
     ref = torch.argmax(x, dim=-1)
     torch.cuda.synchronize()
     assert torch.equal(got, ref), (got[:8].tolist(), ref[:8].tolist())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_large_calls_past_the_caches(gpu, dtype):
+    """From 512 MB of traffic a call-site kernel uses non-temporal loads and
+    stores: the same bits as the same rows in calls below that line."""
+    print(f"case: call-site kernels past the caches {dtype}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(6)
+
+    def rnd(*shape):
+        return torch.empty(shape, dtype=dtype, device=gpu).normal_(generator=g)
+
+    def parts(n, k):
+        at = [n * i // k for i in range(k + 1)]
+        return [slice(a, b) for a, b in zip(at, at[1:])]
+
+    rows, hidden = (1 << 16) + 3, 1024  # 8 bytes an element with the residual
+    x, r, w = rnd(rows, hidden), rnd(rows, hidden), 1 + 0.1 * rnd(hidden)
+    out, res = fz.rmsnorm(x, w, 1e-6, residual=r)
+    for s in parts(rows, 3):
+        o, h = fz.rmsnorm(x[s], w, 1e-6, residual=r[s])
+        assert torch.equal(out[s], o) and torch.equal(res[s], h)
+    rows2 = 2 * rows - 5  # 4 bytes an element without
+    x = rnd(rows2, hidden)
+    out = fz.rmsnorm(x, w, 1e-6)
+    for s in parts(rows2, 3):
+        assert torch.equal(out[s], fz.rmsnorm(x[s], w, 1e-6))
+    del x, r, out, res, o, h
+
+    rows, inter = 29129, 3072  # 6 bytes an element
+    gu = rnd(rows, 2 * inter)
+    act = fz.silu_mul(gu)
+    for s in parts(rows, 3):
+        assert torch.equal(act[s], fz.silu_mul(gu[s]))
+    del gu, act
+
+    T, hq, hkv = 33001, 16, 8  # 16 KB a token, one wavefront each as in its parts
+    qkv, qw, kw = rnd(T, (hq + 2 * hkv) * 128), 1 + 0.1 * rnd(128), 1 + 0.1 * rnd(128)
+    rope = Rope(128, 4096, 1e6, gpu, dtype)
+    pos = torch.randint(0, 4096, (T,), generator=g, device=gpu, dtype=torch.int32)
+    slots = torch.randperm(T + 100, generator=g, device=gpu)[:T]
+    slots[::97] = -1
+    kc, vc, kc2, vc2 = torch.zeros((4, T + 100, hkv, 128), dtype=dtype, device=gpu)
+    q, k = fz.qk_norm_rope_store(qkv, hq, hkv, qw, kw, 1e-6, rope.cos, rope.sin, pos, kc, vc,
+                                 slot_mapping=slots)
+    for s in parts(T, 3):
+        q2, k2 = fz.qk_norm_rope_store(qkv[s], hq, hkv, qw, kw, 1e-6, rope.cos, rope.sin, pos[s],
+                                       kc2, vc2, slot_mapping=slots[s])
+        assert torch.equal(q[s], q2) and torch.equal(k[s], k2)
+    assert torch.equal(kc, kc2) and torch.equal(vc, vc2)

@@ -546,3 +546,59 @@ def test_prefill_few_queries(gpu, hq, hkv, dtype, causal, keys):
         assert torch.equal(kc.view(-1, hkv, 128), ek) and torch.equal(vc.view(-1, hkv, 128), ev)
         if most == 70:
             assert torch.equal(plain, stored)
+
+
+@pytest.mark.parametrize("lens,hq,hkv,store", [
+    ([2401, 1, 130, 37], 32, 8, False),            # long, groups of 4
+    ([513] + [1, 31, 33, 64, 5, 128, 17] * 19, 16, 8, True),   # many items
+    ([513] + [1, 31, 33, 64, 5, 128, 17] * 19, 16, 8, False),
+])
+def test_fp16_on_the_four_wave_kernel(gpu, lens, hq, hkv, store):
+    """The fp16 calls that the four-wave kernel takes: many items and 512 queries,
+    or groups of 4 from 2400 queries on."""
+    print(f"case: fp16 four-wave {hq}/{hkv} {len(lens)} segments store={store}", flush=True)
+    q, k, v, cq, _ = _ragged(lens, lens, hq, hkv, torch.float16, gpu, 34)
+    if store:
+        kc = torch.zeros((sum(lens), hkv, 128), dtype=torch.float16, device=gpu)
+        vc = torch.zeros_like(kc)
+        slots = torch.randperm(sum(lens), device=gpu)
+        out = fai.varlen_prefill_with_kvcache(q, k, v, cq, max(lens), kc, vc, slots, causal=True)
+        torch.cuda.synchronize()
+        assert torch.equal(kc[slots], k) and torch.equal(vc[slots], v)
+    else:
+        out = fai.flash_attn_varlen_func(q, k, v, cq, cq, max(lens), max(lens), causal=True)
+    torch.cuda.synchronize()
+    _oracle_check({"out": out}, q, k, v, cq, cq, True, "fp16 four-wave")
+
+
+@pytest.mark.parametrize("lens,hq,hkv,dtype", [
+    ([257, 129, 33, 777, 1], 16, 8, torch.bfloat16),      # four key slices
+    ([100, 31, 64, 65, 1, 32], 16, 8, torch.bfloat16),     # two key slices
+    ([33, 257, 40, 129, 1] * 30, 16, 8, torch.bfloat16),   # the four-wave kernel
+    ([33, 257, 40, 129, 1] * 30, 16, 8, torch.float16),    # the eight-wave kernel
+    ([257, 129, 33, 300, 1], 8, 8, torch.float16),         # one query head per KV head
+    ([1100, 1000, 33], 8, 8, torch.bfloat16),              # the same, items in two pieces
+])
+@pytest.mark.parametrize("causal", [True, False])
+def test_rows_behind_a_segment_are_not_read_into_it(gpu, lens, hq, hkv, dtype, causal):
+    """K/V rows of the next segment, NaN or infinite, and past the last one do not
+    reach a segment's outputs: loads past its keys give zeros."""
+    print(f"case: NaN rows behind segments {hq}/{hkv} {dtype} causal={causal} {lens[:6]}", flush=True)
+    q, k, v, cq, _ = _ragged(lens + [64], lens + [64], hq, hkv, dtype, gpu, 35)
+    cq = cq[:-1].contiguous()  # the last 64 rows belong to no segment
+    n, M = sum(lens), max(lens)
+    ends = np.concatenate([[0], np.cumsum(lens)])
+    want = fai.flash_attn_varlen_func(q, k, v, cq, cq, M, M, causal=causal)[:n]
+    for odd in (0, 1):
+        kb, vb = k.clone(), v.clone()
+        keep = torch.zeros(n, dtype=torch.bool, device=gpu)
+        for i in range(len(lens)):
+            a, b = int(ends[i]), int(ends[i + 1])
+            if i % 2 == odd:
+                kb[a:b], vb[a:b] = float("nan"), float("inf")
+            else:
+                keep[a:b] = True
+        kb[n:], vb[n:] = float("nan"), float("nan")
+        out = fai.flash_attn_varlen_func(q, kb, vb, cq, cq, M, M, causal=causal)[:n]
+        torch.cuda.synchronize()
+        assert torch.equal(out[keep], want[keep])
