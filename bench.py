@@ -33,8 +33,7 @@ Also reported on the same line:
                 and torch's own flash attention (SDPA, flash backend) on the
                 same shape for reference;
   prefill_one_request  one 2048-token request: too few work items for the
-                CUs, so the keys are split over a workgroup's waves (the
-                same call without a workspace beside it);
+                CUs, so the keys are split over a workgroup's waves;
   prefill_long  the same kernel on 8 x 8192 causal tokens: its steady-state
                 rate, where per-item start and epilogue costs are small;
   prefill_engine  the prefill call the engine makes for 256 fresh 1024-token
@@ -571,9 +570,7 @@ def bench_prefill_engine(torch, fai, paged, dev, args, nseq=256, L=1024, hq=16, 
 
 def bench_prefill_one_request(torch, fai, dev, args, L=2048, hq=16, hkv=8):
     """One 2048-token request (16/8 heads, causal), on the kernel that splits
-    the keys over a workgroup's waves; the same call without a workspace
-    beside it (``us_unsplit``: this kernel needs none)."""
-    from awesome_acceleration_amd import _lib
+    the keys over a workgroup's waves."""
     d = 128
     g = torch.Generator(device=dev).manual_seed(args.seed)
     q = torch.randn((L, hq, d), generator=g, device=dev).to(torch.bfloat16)
@@ -581,28 +578,17 @@ def bench_prefill_one_request(torch, fai, dev, args, L=2048, hq=16, hkv=8):
     v = torch.randn((L, hkv, d), generator=g, device=dev).to(torch.bfloat16)
     cu = torch.tensor([0, L], dtype=torch.int32, device=dev)
     flops = 4 * hq * d * (L * (L + 1) // 2)
-    out = torch.empty_like(q)
-    lib, st = _lib.lib(), torch.cuda.current_stream().cuda_stream
 
-    def split():
+    def attend():
         return fai.flash_attn_varlen_func(q, k, v, cu, cu, L, L, causal=True)
 
-    def unsplit():
-        lib.aac_prefill_varlen(q.data_ptr(), k.data_ptr(), v.data_ptr(), hq * d, hkv * d, hkv * d,
-                               cu.data_ptr(), cu.data_ptr(), 1, L, L, hq, hkv, d, d ** -0.5, 1,
-                               out.data_ptr(), hq * d, None, 0, 0, st)
-
     for _ in range(3):
-        split()
-        unsplit()
-    warm(torch, [split, unsplit], min(args.warmup_seconds, 0.5))
-    t = launch_avg(torch, split, args.steps)
-    t0 = launch_avg(torch, unsplit, args.steps)
-    ws = lib.aac_prefill_workspace_bytes(1, L, L, hq, hkv, d, 1)
+        attend()
+    warm(torch, [attend], min(args.warmup_seconds, 0.5))
+    t = launch_avg(torch, attend, args.steps)
     return {"workload": f"varlen causal prefill of one {L}-token request, {hq}/{hkv} heads, "
                         "head_dim 128, bf16: keys split over each workgroup's waves",
-            "us_attend": round(t * 1e6, 2), "us_unsplit": round(t0 * 1e6, 2),
-            "workspace_bytes": int(ws),
+            "us_attend": round(t * 1e6, 2),
             "roofline": {"bound": "mfma", "achieved": round(flops / t / 1e12, 2),
                          "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                          "frac": round(flops / t / 1e12 / BF16_PEAK_TFLOPS, 4),
